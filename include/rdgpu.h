@@ -363,7 +363,9 @@ enum { RD_KERNEL_AUTO = 0, RD_KERNEL_GATHER = 1, RD_KERNEL_QUEUE = 2 };
 typedef struct {
     int kernel;            /* RD_KERNEL_*: GATHER one lane per particle walks its stencil rows,
                               testing distances first and evaluating the listed hits after, one
-                              workgroup per group of 64-slot work items.  QUEUE: the same per-lane
+                              workgroup per group of 64-slot work items; at 256 threads and one particle
+                              per lane, systems too small to fill the chip (up to 8 work items per
+                              compute unit) take 3 or 9 lanes per particle.  QUEUE: the same per-lane
                               work on a resident grid (occupancy x compute units) whose workgroups
                               each own a contiguous share of the work items, taken by their waves
                               from a ticket in LDS until none are left (ppt is ignored).

@@ -101,11 +101,12 @@ __device__ __forceinline__ uint32_t cell_key(const RdRep& R, float x, float y, f
     return (uint32_t)(R.coff + (cz * R.L[1] + cy) * R.L[0] + cx);
 }
 
-// Visit every slot j of the cells within S of (cx,cy,cz).  Rows along x are
-// contiguous in the sorted arrays, so each row is one or two slot ranges.
+// Visit the slot ranges [j0, j1) that hold the cells within S of (cx,cy,cz):
+// rows along x are contiguous in the sorted arrays, so each row is one or two
+// ranges.
 template <class F>
-__device__ __forceinline__ void for_stencil(const RdRep& R, const uint32_t* __restrict__ start, int cx, int cy,
-                                            int cz, int S, F&& f)
+__device__ __forceinline__ void for_stencil_rows(const RdRep& R, const uint32_t* __restrict__ start, int cx, int cy,
+                                                 int cz, int S, F&& f)
 {
     const int Lx = R.L[0], Ly = R.L[1], Lz = R.L[2];
     int ylo, yhi, zlo, zhi;
@@ -121,14 +122,20 @@ __device__ __forceinline__ void for_stencil(const RdRep& R, const uint32_t* __re
             int yy = fy ? oy : cy + oy;
             if (yy < 0) yy += Ly; else if (yy >= Ly) yy -= Ly;
             int row = R.coff + (zz * Ly + yy) * Lx;
-            uint32_t j0 = start[row + a0], j1 = start[row + b0 + 1];
-            for (uint32_t j = j0; j < j1; ++j) f(j);
-            if (nr == 2) {
-                j0 = start[row + a1]; j1 = start[row + b1 + 1];
-                for (uint32_t j = j0; j < j1; ++j) f(j);
-            }
+            f(start[row + a0], start[row + b0 + 1]);
+            if (nr == 2) f(start[row + a1], start[row + b1 + 1]);
         }
     }
+}
+
+// Visit every slot j of those ranges.
+template <class F>
+__device__ __forceinline__ void for_stencil(const RdRep& R, const uint32_t* __restrict__ start, int cx, int cy,
+                                            int cz, int S, F&& f)
+{
+    for_stencil_rows(R, start, cx, cy, cz, S, [&](uint32_t j0, uint32_t j1) {
+        for (uint32_t j = j0; j < j1; ++j) f(j);
+    });
 }
 
 // for_stencil with each slot's record loaded one slot ahead of its use, so
@@ -372,15 +379,16 @@ __device__ __forceinline__ float3 finish_grad(const RdDev* __restrict__ P, const
 
 // bonded partners of the particle in slot s (group potentials,
 // CudaSimulation.cu:1829-1836): minimum-image distance, no cutoff, added to
-// the fixed-point pair sum
+// the fixed-point pair sum; bonds first, first + stride, ... of the particle
 template <bool ENERGY>
 __device__ __forceinline__ void bond_accum(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
-                                           const float4* __restrict__ ps, float4 p, RdAcc& acc)
+                                           const float4* __restrict__ ps, float4 p, RdAcc& acc, int first = 0,
+                                           int stride = 1)
 {
     const uint32_t gi = (uint32_t)R.off + w_index(p.w);
     const int b1 = P->bstart[gi + 1];
     const int rowbase = w_type(p.w) * P->nt;
-    for (int b = P->bstart[gi]; b < b1; ++b) {
+    for (int b = P->bstart[gi] + first; b < b1; b += stride) {
         const int2 bd = P->bonds[b];
         const float4 q = ps[P->slot_of[bd.x]];
         const float dx = min_image(p.x - q.x, R.Lb[0], R.half[0]);
@@ -632,6 +640,111 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
     return g;
 }
 
+// |minimum image| of a separation: min(|d|, Lb - |d|).  With half = Lb / 2
+// (exact) it equals |min_image(d)| bit for bit while |d| <= Lb, at two
+// instructions, and a range test needs only the magnitude.
+__device__ __forceinline__ float min_image_abs(float d, float Lb) { return fminf(fabsf(d), Lb - fabsf(d)); }
+
+// Pair and bond terms of the particle in slot s shared by G lanes (sub = 0 ..
+// G-1 of the particle): lane sub walks the stencil rows sub, sub + G, ... and
+// adds its terms to acc; the lanes' sums are then added (integers: the same
+// bits in any split).  Each lane loads up to four candidates of a run at
+// once, and lists the separation and type of those in range in LDS, so that
+// the evaluation reads no record again.
+#define RD_ROW_HITS 4
+struct RdRowHit {
+    float dx, dy, dz;
+    int tj;
+};
+
+template <bool ENERGY, int G>
+__device__ __forceinline__ void gather_rows(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
+                                            const float4* __restrict__ ps, const uint32_t* __restrict__ start,
+                                            uint32_t s, float4 p, int sub, RdAcc& acc, RdRowHit (*__restrict__ il)[64])
+{
+    constexpr int NR = (9 + G - 1) / G;
+    const int rowbase = w_type(p.w) * P->nt;
+    const int lane = threadIdx.x & 63;
+    const int Lx = R.L[0], Ly = R.L[1], Lz = R.L[2];
+    if (P->n_pot2 > 0) {
+        int cx, cy, cz;
+        cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
+        if (P->S == 1 && Lx >= 3 && Ly >= 3 && Lz >= 3) {
+            int a0, b0, a1 = 0, b1 = -1;
+            const int nr = x_runs(cx, 1, Lx, &a0, &b0, &a1, &b1);
+            // bounds of the lane's rows (first runs, then second runs), all
+            // loads in flight at once
+            uint32_t jb[2 * NR], je[2 * NR];
+#pragma unroll
+            for (int k = 0; k < NR; ++k) {
+                const int r = sub + k * G;
+                int yy = cy + (r % 3) - 1, zz = cz + (r / 3) - 1;
+                yy += yy < 0 ? Ly : 0; yy -= yy >= Ly ? Ly : 0;
+                zz += zz < 0 ? Lz : 0; zz -= zz >= Lz ? Lz : 0;
+                const int row = R.coff + (zz * Ly + yy) * Lx;
+                jb[k] = je[k] = jb[NR + k] = je[NR + k] = 0u;
+                if (r < 9) {
+                    jb[k] = start[row + a0];
+                    je[k] = start[row + b0 + 1];
+                    if (nr == 2) {
+                        jb[NR + k] = start[row + a1];
+                        je[NR + k] = start[row + b1 + 1];
+                    }
+                }
+            }
+            int nhit = 0;
+            auto eval = [&](float dx, float dy, float dz, int tj) {
+                dx = min_image(dx, R.Lb[0], R.half[0]);
+                dy = min_image(dy, R.Lb[1], R.half[1]);
+                dz = min_image(dz, R.Lb[2], R.half[2]);
+                pair_add<ENERGY, true>(T, rowbase, dx, dy, dz, dist2(dx, dy, dz), tj, acc);
+            };
+            // candidates in range are listed; past the list they are
+            // evaluated as they are met
+            auto test = [&](float4 q) {
+                const float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+                const int tj = w_type(q.w);
+                const float d2 = dist2(min_image_abs(dx, R.Lb[0]), min_image_abs(dy, R.Lb[1]),
+                                       min_image_abs(dz, R.Lb[2]));
+                if (d2 < T.rc2[rowbase + tj] && d2 > 0.0f) {
+                    if (nhit < RD_ROW_HITS) {
+                        il[nhit][lane] = { dx, dy, dz, tj };
+                        ++nhit;
+                    } else {
+                        eval(dx, dy, dz, tj);
+                    }
+                }
+            };
+#pragma unroll
+            for (int k = 0; k < 2 * NR; ++k) {
+                const uint32_t e = je[k];
+                for (uint32_t j = jb[k]; j < e; j += 4) {
+                    const uint32_t l = e - 1u;
+                    const float4 q0 = ps[j], q1 = ps[min(j + 1u, l)], q2 = ps[min(j + 2u, l)], q3 = ps[min(j + 3u, l)];
+                    test(q0);
+                    if (j + 1u < e) test(q1);
+                    if (j + 2u < e) test(q2);
+                    if (j + 3u < e) test(q3);
+                }
+            }
+            for (int k = 0; __any(k < nhit); ++k)
+                if (k < nhit) {
+                    const RdRowHit h = il[k][lane];
+                    eval(h.dx, h.dy, h.dz, h.tj);
+                }
+        } else {
+            // any other stencil: its rows dealt to the lanes in turn
+            int row = 0;
+            for_stencil_rows(R, start, cx, cy, cz, P->S, [&](uint32_t j0, uint32_t j1) {
+                if (row++ % G == sub)
+                    for (uint32_t j = j0; j < j1; ++j)
+                        if (j != s) pair_accum<ENERGY>(T, rowbase, p, ps[j], R, acc);
+            });
+        }
+    }
+    if (P->bstart) bond_accum<ENERGY>(P, R, T, ps, p, acc, sub, G);
+}
+
 __device__ __forceinline__ float wrap_coord(float x, float lo, float hi, float Lb)
 {
     if (x > hi) x -= Lb;
@@ -639,37 +752,38 @@ __device__ __forceinline__ float wrap_coord(float x, float lo, float hi, float L
     return x;
 }
 
-// Euler-Maruyama for slot s (CudaSimulation.cu:1850-1858): noise, x += -a*dU
+// noise of slot s's particle in this step: the generator, or the
+// caller-supplied array (indexed by the global particle index; outside its
+// steps: zero, and RD_ERR_NOISE).  The noise counter is (local index, step,
+// replica stream).
+__device__ __forceinline__ float3 step_noise(const RdDev* __restrict__ P, const RdRep& R, RdStepState* __restrict__ st,
+                                             const float* __restrict__ noise, int ntot, uint32_t idx)
+{
+    const unsigned long long step = st->step;
+    if (st->noise_nsteps == 0) return rd_normal3(P->seed, R.stream, step, idx);
+    const long long ls = (long long)(step - st->noise_step0);
+    if (ls >= 0 && ls < st->noise_nsteps) {
+        const size_t base = (size_t)ls * 3 * (size_t)ntot + (size_t)R.off + idx;
+        return make_float3(noise[base], noise[base + ntot], noise[base + 2 * (size_t)ntot]);
+    }
+    atomicOr(&st->err, RD_ERR_NOISE);
+    return make_float3(0.0f, 0.0f, 0.0f);
+}
+
+// Euler-Maruyama for slot s (CudaSimulation.cu:1850-1858): x += -a*dU
 // + b*xi, one periodic correction, the next cell key and its histogram entry.
 // The reference repeats the correction until the particle is inside
 // (:1857-1858); a particle that is still outside after one correction moved
 // more than a box length in one step, which is reported as an error
-// (RD_ERR_OUTSIDE) rather than wrapped.  The noise counter is (local index,
-// step, replica stream); a caller-supplied noise array is indexed by the
-// global particle index.
+// (RD_ERR_OUTSIDE) rather than wrapped.
 __device__ __forceinline__ void em_update_store(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
-                                                RdStepState* __restrict__ st, const float* __restrict__ noise,
-                                                int ntot, uint32_t s, float4 p, float3 g, bool sat,
-                                                float4* __restrict__ pn,
+                                                RdStepState* __restrict__ st, uint32_t s, float4 p, float3 g, float3 z,
+                                                bool sat, float4* __restrict__ pn,
                                                 uint2* __restrict__ kr,
                                                 uint32_t* __restrict__ count, uint32_t* __restrict__ tsum)
 {
     const int t = w_type(p.w);
     const uint32_t idx = w_index(p.w);
-    const unsigned long long step = st->step;
-    float3 z;
-    if (st->noise_nsteps == 0) {
-        z = rd_normal3(P->seed, R.stream, step, idx);
-    } else {
-        long long ls = (long long)(step - st->noise_step0);
-        if (ls >= 0 && ls < st->noise_nsteps) {
-            size_t base = (size_t)ls * 3 * (size_t)ntot + (size_t)R.off + idx;
-            z = make_float3(noise[base], noise[base + ntot], noise[base + 2 * (size_t)ntot]);
-        } else {
-            z = make_float3(0.0f, 0.0f, 0.0f);
-            atomicOr(&st->err, RD_ERR_NOISE);
-        }
-    }
     const float a = T.a[t], bb = T.b[t];
     float x = (p.x - a * g.x) + bb * z.x;
     float y = (p.y - a * g.y) + bb * z.y;

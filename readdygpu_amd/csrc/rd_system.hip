@@ -73,7 +73,7 @@ __device__ __forceinline__ void force_update(RD_FORCE_ARGS)
         const RdRep R = reps[it.rep];
         bool sat;
         float3 g = gather_grad<false>(P, R, T, pot1, ps, start, s, p, nullptr, &sat, &il[threadIdx.x >> 6]);
-        em_update_store(P, R, T, st, noise, ntot, s, p, g, sat, pn, kr, count, tsum);
+        em_update_store(P, R, T, st, s, p, g, step_noise(P, R, st, noise, ntot, w_index(p.w)), sat, pn, kr, count, tsum);
     } else {
         load_tab<BLOCK>(T, P);
         for (int k = 0; k < PPT; ++k) {
@@ -84,7 +84,7 @@ __device__ __forceinline__ void force_update(RD_FORCE_ARGS)
                 float4 p = ps[s];
                 bool sat;
                 float3 g = gather_grad<false>(P, R, T, pot1, ps, start, s, p, nullptr, &sat, &il[threadIdx.x >> 6]);
-                em_update_store(P, R, T, st, noise, ntot, s, p, g, sat, pn, kr, count, tsum);
+                em_update_store(P, R, T, st, s, p, g, step_noise(P, R, st, noise, ntot, w_index(p.w)), sat, pn, kr, count, tsum);
             }
         }
     }
@@ -139,9 +139,94 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void
             const float4 p = ps[s];
             bool sat;
             const float3 g = gather_grad<false>(P, R, T, pot1, ps, start, s, p, nullptr, &sat, &il[threadIdx.x >> 6]);
-            em_update_store(P, R, T, st, noise, ntot, s, p, g, sat, pn, kr, count, tsum);
+            em_update_store(P, R, T, st, s, p, g, step_noise(P, R, st, noise, ntot, w_index(p.w)), sat, pn, kr, count, tsum);
         }
     }
+}
+
+// Sums of the particles of a workgroup in LDS, added to by the lanes that
+// share a particle.
+template <bool ENERGY>
+struct RdShared {       // fixed-point sums, energies, range flags
+    unsigned long long f[64][3];
+    double e[ENERGY ? 64 : 1];
+    uint32_t sat[64];
+};
+
+// One 64-slot work item per workgroup of G + 1 waves: the first G waves walk
+// with G lanes per particle (gather_rows); the last one holds one particle per
+// lane, computes the noise meanwhile and afterwards updates its particle with
+// the sums.
+template <bool ENERGY, int G>
+__device__ __forceinline__ void spread_walk(const float4* __restrict__ ps, const uint32_t* __restrict__ start,
+                                            const RdDev* __restrict__ P, const RdRep* __restrict__ reps, RdWave it,
+                                            const RdTab& T, float4 p, RdShared<ENERGY>& S,
+                                            RdRowHit (*__restrict__ il)[RD_ROW_HITS][64])
+{
+    const int i = (int)threadIdx.x / G;
+    const uint32_t s = (uint32_t)(it.s0 + i);
+    if (s >= (uint32_t)it.s1) return;
+    const RdRep R = reps[it.rep];
+    RdAcc a;
+    a.x = 0; a.y = 0; a.z = 0; a.e = 0.0; a.sat = false;
+    gather_rows<ENERGY, G>(P, R, T, ps, start, s, p, (int)threadIdx.x % G, a, il[threadIdx.x >> 6]);
+    if (a.x != 0) atomicAdd(&S.f[i][0], (unsigned long long)a.x);
+    if (a.y != 0) atomicAdd(&S.f[i][1], (unsigned long long)a.y);
+    if (a.z != 0) atomicAdd(&S.f[i][2], (unsigned long long)a.z);
+    if (a.sat) atomicOr(&S.sat[i], 1u);
+    if (ENERGY && a.e != 0.0) atomicAdd(&S.e[i], a.e);
+}
+
+template <bool ENERGY>
+__device__ __forceinline__ void shared_clear(RdShared<ENERGY>& S)
+{
+    const int t = threadIdx.x;
+    if (t < 64) {
+        S.f[t][0] = S.f[t][1] = S.f[t][2] = 0ull;
+        S.sat[t] = 0u;
+        if (ENERGY) S.e[t] = 0.0;
+    }
+}
+
+// The step of a small system with G lanes per particle (9: one stencil row per
+// lane; 3: three).  Bound by the latency of its chain of dependent loads
+// (record, run bounds, candidates, then the histogram's atomic): 9.9 us for
+// 10,000 particles against 27.4 us with one lane per particle, whose chain
+// runs through all nine rows.
+template <int G>
+__global__ __launch_bounds__(64 * (G + 1)) void k_force_update_spread(RD_FORCE_ARGS, int nrep)
+{
+    __shared__ RdTab T;
+    __shared__ RdRowHit il[G][RD_ROW_HITS][64];
+    __shared__ RdShared<false> S;
+    const int w = xcd_block(blockIdx.x, gridDim.x);
+    RdWave it;
+    if (nrep == 1) {             // the work item without a load
+        it.rep = 0; it.s0 = 64 * w; it.s1 = min(ntot, 64 * w + 64); it.pad = 0;
+    } else {
+        it = wave_item(waves, nwaves, w);
+    }
+    const bool walker = threadIdx.x < 64 * G;
+    const uint32_t s = (uint32_t)(it.s0 + (walker ? (int)threadIdx.x / G : (int)threadIdx.x - 64 * G));
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (s < (uint32_t)it.s1) p = ps[s];
+    shared_clear<false>(S);
+    load_tab<64 * (G + 1)>(T, P);                // ends with a workgroup barrier
+    float3 z = make_float3(0.0f, 0.0f, 0.0f);
+    if (walker) spread_walk<false, G>(ps, start, P, reps, it, T, p, S, il);
+    else if (s < (uint32_t)it.s1) z = step_noise(P, reps[it.rep], st, noise, ntot, w_index(p.w));
+    __syncthreads();
+    if (walker || s >= (uint32_t)it.s1) return;
+    const RdRep R = reps[it.rep];
+    const int i = (int)threadIdx.x - 64 * G;
+    RdAcc acc;
+    acc.x = (long long)S.f[i][0];
+    acc.y = (long long)S.f[i][1];
+    acc.z = (long long)S.f[i][2];
+    acc.sat = S.sat[i] != 0u;
+    acc.e = 0.0;
+    const float3 g = finish_grad<false>(P, T, pot1, s, p, acc, nullptr);
+    em_update_store(P, R, T, st, s, p, g, z, acc.sat, pn, kr, count, tsum);
 }
 
 // gradient + energy (FP64 accumulation) at the current positions
@@ -180,6 +265,48 @@ __global__ __launch_bounds__(RD_BLOCK) void k_gradients(const float4* __restrict
         for (int w = 0; w < RD_BLOCK / 64; ++w) t += red[w];
         atomicAdd(etot, t);
     }
+}
+
+// the same for small systems, G lanes per particle (as k_force_update_spread)
+template <int G>
+__global__ __launch_bounds__(64 * G) void k_gradients_spread(const float4* __restrict__ ps,
+                                                             const uint32_t* __restrict__ start,
+                                                             const RdDev* __restrict__ P,
+                                                             const RdRep* __restrict__ reps,
+                                                             const RdWave* __restrict__ waves, int nwaves,
+                                                             const RdPot1Dev* __restrict__ pot1,
+                                                             float* __restrict__ grad, double* __restrict__ etot,
+                                                             RdStepState* __restrict__ st)
+{
+    __shared__ RdTab T;
+    __shared__ RdRowHit il[G][RD_ROW_HITS][64];
+    __shared__ RdShared<true> S;
+    const RdWave it = wave_item(waves, nwaves, xcd_block(blockIdx.x, gridDim.x));
+    const uint32_t sw = (uint32_t)(it.s0 + (int)threadIdx.x / G), s = (uint32_t)(it.s0 + (int)threadIdx.x);
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q = p;
+    if (sw < (uint32_t)it.s1) q = ps[sw];
+    if (threadIdx.x < 64 && s < (uint32_t)it.s1) p = ps[s];
+    shared_clear<true>(S);
+    load_tab<64 * G>(T, P);                      // ends with a workgroup barrier
+    spread_walk<true, G>(ps, start, P, reps, it, T, q, S, il);
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double e = 0.0;
+    if (s < (uint32_t)it.s1) {
+        const int i = (int)threadIdx.x;
+        RdAcc acc;
+        acc.x = (long long)S.f[i][0];
+        acc.y = (long long)S.f[i][1];
+        acc.z = (long long)S.f[i][2];
+        e = S.e[i];
+        const float3 g = finish_grad<true>(P, T, pot1, s, p, acc, &e);
+        if (S.sat[i] != 0u) atomicOr(&st->err, RD_ERR_FIXRANGE);
+        const size_t gi = (size_t)reps[it.rep].off + w_index(p.w);
+        grad[3 * gi] = g.x; grad[3 * gi + 1] = g.y; grad[3 * gi + 2] = g.z;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o, 64);
+    if (threadIdx.x == 0) atomicAdd(etot, e);
 }
 
 // ---- exclusive scan of count[ncell] -> start[ncell+1], zeroing count ----
@@ -1299,6 +1426,37 @@ static void launch_force_queue(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
                            h->d_st, h->d_noise, h->n);
 }
 
+// Lanes per particle of the default launch shape (256 threads, one particle
+// per lane asked for): 9 or 3 while every 64-slot work item still runs in one
+// round of resident workgroups (640 threads: 3 per CU; 256 threads: 8 per CU),
+// 1 beyond.  Below that line a step's time is one lane's chain of dependent
+// loads, which the split shortens; above it the split only repeats the
+// per-workgroup work.  Whole step, 1 / 3 / 9 lanes (us): 2,000 particles
+// 22.9 / 13.0 / 11.3, 10,000 32.0 / 16.7 / 14.1, 30,000 50.3 / 31.8 / 24.8,
+// 50,000 24.8 / 20.9 / 22.2 (sparser), 100,000 29.2 / 27.2 / 32.8,
+// 200,000 37.8 / 39.6 / 57.0.
+static int lanes_per_particle(const rd_system* h)
+{
+    if (h->kern != RD_KERNEL_GATHER || h->block != 256 || h->ppt != 1) return 1;
+    return h->nwaves <= 3 * h->ncu ? 9 : h->nwaves <= 8 * h->ncu ? 3 : 1;
+}
+
+template <int G>
+static void launch_force_spread(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
+{
+    const dim3 grid(std::max(1, h->nwaves));
+    if (ev0)
+        hipExtLaunchKernelGGL((k_force_update_spread<G>), grid, dim3(64 * (G + 1)), 0, h->stream, ev0, ev1, 0,
+                              (const float4*)h->d_ps, h->d_pn, h->d_kr, h->d_count, h->d_bsum,
+                              (const uint32_t*)h->d_start, (const RdDev*)h->d_P, (const RdRep*)h->d_reps,
+                              (const RdWave*)h->d_waves, h->nwaves, (const RdPot1Dev*)h->d_pot1, h->d_st,
+                              (const float*)h->d_noise, h->n, (int)h->rep_dev.size());
+    else
+        hipLaunchKernelGGL((k_force_update_spread<G>), grid, dim3(64 * (G + 1)), 0, h->stream, h->d_ps, h->d_pn, h->d_kr,
+                           h->d_count, h->d_bsum, h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1,
+                           h->d_st, h->d_noise, h->n, (int)h->rep_dev.size());
+}
+
 template <int B>
 static void launch_force_ppt(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 {
@@ -1316,6 +1474,11 @@ static void launch_force_ppt(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 void rd_host_launch_force(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 {
     if (h->n <= 0) return;
+    switch (lanes_per_particle(h)) {
+    case 9: launch_force_spread<9>(h, ev0, ev1); return;
+    case 3: launch_force_spread<3>(h, ev0, ev1); return;
+    default: break;
+    }
     switch (h->block) {
     case 64: launch_force_ppt<64>(h, ev0, ev1); break;
     case 128: launch_force_ppt<128>(h, ev0, ev1); break;
@@ -1615,7 +1778,12 @@ extern "C" int rd_gradients(rd_system* h, float* grad, double* energy)
     if (h->n == 0) { if (energy) *energy = 0.0; return RD_OK; }
     HIPCK(h, hipMemsetAsync(h->d_etot, 0, sizeof(double), h->stream));
     if (h->ext_active()) rd_host_launch_ext(h);
-    hipLaunchKernelGGL(k_gradients, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_start, h->d_P,
+    if (h->nwaves <= 3 * h->ncu)     // the line of lanes_per_particle
+        hipLaunchKernelGGL((k_gradients_spread<9>), dim3(std::max(1, h->nwaves)), dim3(64 * 9), 0, h->stream, h->d_ps,
+                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, h->d_etot,
+                           h->d_st);
+    else
+        hipLaunchKernelGGL(k_gradients, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_start, h->d_P,
                            h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, h->d_etot, h->d_st);
     HIPCK(h, hipGetLastError());
     std::vector<float> tmp(3 * (size_t)h->n);
