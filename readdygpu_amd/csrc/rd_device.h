@@ -48,7 +48,8 @@ struct RdRep {
 
 // one wave of work: 64 consecutive slots of one replica
 struct RdWave {
-    int rep, s0, s1, pad;
+    int rep, s0, s1;
+    int next;           // first work item of the next replica
 };
 
 // per-system constants, read through one pointer (scalar loads)
@@ -104,6 +105,12 @@ __device__ __forceinline__ float min_image(float d, float Lb, float h)
     if (d < -h) d += Lb;
     return d;
 }
+
+// |minimum image| of a separation: min(|d|, Lb - |d|).  With half = Lb / 2
+// (exact) it equals |min_image(d)| bit for bit while |d| <= Lb (any two
+// positions inside the box), at two instructions instead of six; a squared
+// distance needs only the magnitudes.
+__device__ __forceinline__ float min_image_abs(float d, float Lb) { return fminf(fabsf(d), Lb - fabsf(d)); }
 
 // ---------------------------------------------------------------------------
 // Noise: Philox4x32-10 (Salmon et al., SC'11) + Box-Muller with an in-house

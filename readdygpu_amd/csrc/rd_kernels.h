@@ -175,40 +175,105 @@ __device__ __forceinline__ void for_stencil_q(const RdRep& R, const uint32_t* __
     }
 }
 
-// for_stencil_q over the half of the stencil that holds each unordered pair
-// once: the rows (dy, dz) with dz > 0, or dz == 0 and dy > 0, in full, and of
-// the home row the slots after s.  The mirror image of every other row is
-// left out, so a pair is met from exactly one of its two particles.  Needs
-// 2S+1 < L in every dimension (no stencil row is its own mirror image).
-template <class F>
-__device__ __forceinline__ void for_stencil_half_q(const RdRep& R, const uint32_t* __restrict__ start,
-                                                   const float4* __restrict__ ps, uint32_t s, int cx, int cy, int cz,
-                                                   int S, F&& f)
+// Visit each unordered pair of the particle p in slot s that may lie within
+// `reach` once, its stencil rows shared by G lanes (lane sub takes rows sub,
+// sub + G, ...): f(q) with the partner's record.  Where 2S+1 < L in every
+// dimension (no stencil row is its own mirror image) the rows are the half of
+// the stencil that meets a pair from one of its two particles: (dy, dz) with
+// dz > 0, or dz = 0 and dy > 0, in full, and of the home row the slots after
+// s.  Each such row is cut to the cells that the ball of radius reach around
+// the particle touches: with reach 3.3 cells and S = 4, 45% of the cube.  On
+// smaller lattices the rows are all rows, uncut, with the slots after s.  The
+// next row's bounds are loaded while a row is walked, and W records at a time.
+//
+// Cell m of an axis (unwrapped index, position y relative to the box) covers
+// [m c, (m+1) c), except that cell 0 also holds the partial slab of width
+// d = Lb - L c at the top of the box, [-d, 0): cells below are shifted by -d
+// and cells from L on by +d.  The distance to a cell beyond either edge is
+// therefore reduced by d, a particle of the slab is taken at y - Lb, and
+// floor() of a coordinate beyond an edge errs outwards.
+template <int G, int W, class F>
+__device__ __forceinline__ void for_pairs_once(const RdRep& R, const uint32_t* __restrict__ start,
+                                               const float4* __restrict__ ps, uint32_t s, float4 p, int S, float reach,
+                                               int sub, F&& f)
 {
-    auto run = [&](uint32_t j, uint32_t j1) {
-        if (j >= j1) return;
-        float4 q = ps[j];
-        for (; j + 1 < j1; ++j) {
-            const float4 n = ps[j + 1];
-            f(j, q);
-            q = n;
-        }
-        f(j, q);
-    };
     const int Lx = R.L[0], Ly = R.L[1], Lz = R.L[2];
-    int a0, b0, a1, b1;
-    const int nr = x_runs(cx, S, Lx, &a0, &b0, &a1, &b1);
-    for (int oz = 0; oz <= S; ++oz) {
-        int zz = cz + oz;
-        if (zz >= Lz) zz -= Lz;
-        for (int oy = oz == 0 ? 0 : -S; oy <= S; ++oy) {
-            int yy = cy + oy;
-            if (yy < 0) yy += Ly; else if (yy >= Ly) yy -= Ly;
-            const int row = R.coff + (zz * Ly + yy) * Lx;
-            const uint32_t lo = (oz == 0 && oy == 0) ? s + 1u : 0u;
-            run(max(start[row + a0], lo), start[row + b0 + 1]);
-            if (nr == 2) run(max(start[row + a1], lo), start[row + b1 + 1]);
+    const bool half = 2 * S + 1 < Lx && 2 * S + 1 < Ly && 2 * S + 1 < Lz;
+    const bool fy = 2 * S + 1 >= Ly, fz = 2 * S + 1 >= Lz;
+    const int ylo = fy ? 0 : -S, yhi = fy ? Ly - 1 : S, ny = yhi - ylo + 1;
+    const int zhi = fz ? Lz - 1 : S;
+    int cx, cy, cz;
+    cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
+    const float c = R.cell, ic = __builtin_amdgcn_rcpf(c);
+    float px = p.x - R.lo[0], py = p.y - R.lo[1], pz = p.z - R.lo[2];
+    px -= cx == 0 && px > R.half[0] ? R.Lb[0] : 0.0f;
+    py -= cy == 0 && py > R.half[1] ? R.Lb[1] : 0.0f;
+    pz -= cz == 0 && pz > R.half[2] ? R.Lb[2] : 0.0f;
+    // rounding of positions, of the cell index and of these distances
+    const float slack = 1e-3f * c + 2e-6f * fmaxf(R.Lb[0], fmaxf(R.Lb[1], R.Lb[2]));
+    auto gap = [&](int m, float y, float Lb, int L) {
+        float e = fmaxf((float)m * c - y, y - (float)(m + 1) * c) - slack;
+        e -= m <= 0 || m >= L ? Lb - (float)L * c : 0.0f;
+        return fmaxf(e, 0.0f);
+    };
+    int oz = half || fz ? 0 : -S, oy = (half ? 0 : ylo) + sub;
+    int a0, b0, a1 = 0, b1 = -1;
+    int nr = x_runs(cx, S, Lx, &a0, &b0, &a1, &b1);
+    uint32_t n0, n1, m0 = 0u, m1 = 0u;           // first and second run of the next row
+    float rz2 = 0.0f;                            // reach^2 less the z distance of the current rows
+    int zrow = 0;
+    auto plane = [&]() {
+        const float gz = gap(cz + oz, pz, R.Lb[2], Lz);
+        rz2 = reach * reach - gz * gz;
+        int zz = fz ? oz : cz + oz;
+        zz += zz < 0 ? Lz : 0; zz -= zz >= Lz ? Lz : 0;
+        zrow = zz * Ly;
+    };
+    plane();
+    auto load = [&]() {                          // rows past the last or out of reach: no slots
+        if (oy > yhi) {
+            do { oy -= ny; ++oz; } while (oy > yhi);
+            plane();
         }
+        n0 = n1 = m0 = m1 = 0u;
+        if (oz > zhi) return;
+        if (half) {
+            const float gy = gap(cy + oy, py, R.Lb[1], Ly);
+            const float w2 = rz2 - gy * gy;
+            if (!(w2 > 0.0f)) return;
+            const float w = __builtin_amdgcn_sqrtf(w2) + slack;
+            const int ml = min(cx, max(cx - S, (int)floorf((px - w) * ic)));
+            const int mr = max(cx, min(cx + S, (int)floorf((px + w) * ic)));
+            a0 = max(ml, 0); b0 = min(mr, Lx - 1);
+            nr = ml < 0 || mr >= Lx ? 2 : 1;
+            a1 = ml < 0 ? Lx + ml : 0;
+            b1 = ml < 0 ? Lx - 1 : mr - Lx;
+        }
+        int yy = fy ? oy : cy + oy;
+        yy += yy < 0 ? Ly : 0; yy -= yy >= Ly ? Ly : 0;
+        const int row = R.coff + (zrow + yy) * Lx;
+        n0 = start[row + a0];
+        n1 = start[row + b0 + 1];
+        if (nr == 2) { m0 = start[row + a1]; m1 = start[row + b1 + 1]; }
+        if (!half || (oz == 0 && oy == 0)) { n0 = max(n0, s + 1u); m0 = max(m0, s + 1u); }
+    };
+    auto walk = [&](uint32_t j, uint32_t e) {
+        for (; j < e; j += W) {
+            float4 q[W];
+#pragma unroll
+            for (int k = 0; k < W; ++k) q[k] = ps[min(j + (uint32_t)k, e - 1u)];
+#pragma unroll
+            for (int k = 0; k < W; ++k)
+                if (j + (uint32_t)k < e) f(q[k]);
+        }
+    };
+    load();
+    while (oz <= zhi) {
+        const uint32_t c0 = n0, c1 = n1, d0 = m0, d1 = m1;
+        oy += G;
+        load();
+        walk(c0, c1);
+        walk(d0, d1);
     }
 }
 
@@ -640,11 +705,6 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
     return g;
 }
 
-// |minimum image| of a separation: min(|d|, Lb - |d|).  With half = Lb / 2
-// (exact) it equals |min_image(d)| bit for bit while |d| <= Lb, at two
-// instructions, and a range test needs only the magnitude.
-__device__ __forceinline__ float min_image_abs(float d, float Lb) { return fminf(fabsf(d), Lb - fabsf(d)); }
-
 // Pair and bond terms of the particle in slot s shared by G lanes (sub = 0 ..
 // G-1 of the particle): lane sub walks the stencil rows sub, sub + G, ... and
 // adds its terms to acc; the lanes' sums are then added (integers: the same
@@ -808,6 +868,6 @@ __device__ __forceinline__ RdWave wave_item(const RdWave* __restrict__ waves, in
 {
     RdWave it;
     if (w < nwaves) it = waves[w];
-    else { it.rep = 0; it.s0 = 0; it.s1 = 0; it.pad = 0; }
+    else { it.rep = 0; it.s0 = 0; it.s1 = 0; it.next = nwaves; }
     return it;
 }

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(64 * (G + 1)) void k_force_update_spread(RD_FORCE_A
     const int w = xcd_block(blockIdx.x, gridDim.x);
     RdWave it;
     if (nrep == 1) {             // the work item without a load
-        it.rep = 0; it.s0 = 64 * w; it.s1 = min(ntot, 64 * w + 64); it.pad = 0;
+        it.rep = 0; it.s0 = 64 * w; it.s1 = min(ntot, 64 * w + 64); it.next = nwaves;
     } else {
         it = wave_item(waves, nwaves, w);
     }
@@ -618,162 +618,139 @@ __global__ __launch_bounds__(RD_BLOCK) void k_noise_fill(const RdDev* __restrict
     out[base] = z.x; out[base + ntot] = z.y; out[base + 2 * (size_t)ntot] = z.z;
 }
 
-// RDF histogram (CudaSimulation.cu:1784-1827 counts every ordered pair once
-// per side; here each slot counts its own partners).
-// counts[((rep*nt + ti)*nt + tj)*nbins + bin]
-// Candidates with d2 >= rcut2 are skipped before the square root: rcut2 is
-// rmax^2 rounded up by 1e-6 relative, and sqrtf is correctly rounded, so every
-// skipped candidate has sqrtf(d2) >= rmax and the counted set is unchanged.
-// `wrap` false: the home cell's stencil neither wraps nor touches cell 0
-// (which also holds the partial slab at the top of the box), and it spans
-// less than half the box, so every raw difference is already its minimum
-// image (min_image would return it unchanged).
-// bin of the pair (p, q), or -1 beyond rmax
-__device__ __forceinline__ int rdf_bin(const RdRep& R, float4 p, float4 q, float rmax, float rcut2, int nbins,
-                                       bool wrap)
+// squared minimum-image distance in the FP32 operation order of the pair sets
+// and the RDF
+__device__ __forceinline__ float set_dist2(const RdRep& R, float4 p, float4 q)
 {
-    float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-    if (wrap) {
-        dx = min_image(dx, R.Lb[0], R.half[0]);
-        dy = min_image(dy, R.Lb[1], R.half[1]);
-        dz = min_image(dz, R.Lb[2], R.half[2]);
-    }
+    const float dx = min_image_abs(p.x - q.x, R.Lb[0]);
+    const float dy = min_image_abs(p.y - q.y, R.Lb[1]);
+    const float dz = min_image_abs(p.z - q.z, R.Lb[2]);
     float d2 = dx * dx;
     d2 = d2 + dy * dy;
     d2 = d2 + dz * dz;
-    if (!(d2 < rcut2)) return -1;
-    float r = sqrtf(d2);
-    if (!(r < rmax)) return -1;
-    int bin = (int)floorf((r * (float)nbins) / rmax);
-    if (bin > nbins - 1) bin = nbins - 1;
+    return d2;
+}
+
+// RDF histogram (CudaSimulation.cu:1784-1827 counts every ordered pair once
+// per side).  counts[((rep*nt + ti)*nt + tj)*nbins + bin]
+struct RdRdf {
+    float rmax, rcut2;      // rcut2: rmax^2 rounded up by 1e-6 relative
+    int nbins;
+    float scale, margin;    // nbins / rmax; 1e-6 nbins
+};
+
+// bin of a squared distance, floor((sqrt(d2) nbins) / rmax) with IEEE square
+// root and division, or -1 beyond rmax.  The hardware square root times
+// nbins / rmax is within 4.5e-7 nbins of that quotient (1 ulp, two roundings
+// and the constant's against three roundings), so its integer part is the bin
+// unless it lies within the margin of an integer; only then (1 in 2,500
+// distances at 200 bins) the IEEE sequence, about 25 instructions, is run.
+__device__ __forceinline__ int rdf_bin(const RdRdf& rdf, float d2)
+{
+    if (!(d2 < rdf.rcut2)) return -1;
+    const float t = __builtin_amdgcn_sqrtf(d2) * rdf.scale;
+    int bin = (int)t;
+    const float f = t - (float)bin;
+    if (f < rdf.margin || f > 1.0f - rdf.margin || bin >= rdf.nbins) {
+        const float r = sqrtf(d2);
+        if (!(r < rdf.rmax)) return -1;
+        bin = (int)floorf((r * (float)rdf.nbins) / rdf.rmax);
+        if (bin > rdf.nbins - 1) bin = rdf.nbins - 1;
+    }
     return bin;
 }
 
-__device__ __forceinline__ bool stencil_wraps(const RdRep& R, int cx, int cy, int cz, int S)
+// One LDS histogram per workgroup, which takes BLOCK / G / 64 work items, one
+// replica at a time, and adds its histogram to copy b % ncopy of the counts
+// after each replica.  Each unordered pair is counted once, at (type of one
+// particle, type of the other); k_rdf_fold adds the two orders.  G lanes share
+// a particle's rows (W candidates loaded at once).  Bound by issue and the
+// divergence of the row walk (the atomics and flushes are 7 of 200 us at 1M
+// particles).  One round of resident workgroups with contiguous shares of the
+// items was 40% slower at 1M: the dense shell's share takes longest.
+template <int BLOCK, int G, int W>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_rdf_lds(const float4* __restrict__ ps, const uint32_t* __restrict__ start,
+                                                   const RdDev* __restrict__ P, const RdRep* __restrict__ reps,
+                                                   const RdWave* __restrict__ waves, int nwaves, int S, RdRdf rdf,
+                                                   unsigned long long* __restrict__ part, long part_stride, int ncopy)
 {
-    const int L[3] = { R.L[0], R.L[1], R.L[2] }, c[3] = { cx, cy, cz };
-    for (int d = 0; d < 3; ++d)
-        if (c[d] < S + 1 || c[d] > L[d] - 1 - S || (float)(S + 2) * R.cell >= R.half[d]) return true;
-    return false;
-}
-
-// Visits every pair of the particle in slot s with the RDF histogram index
-// of each direction in which the full-stencil count (every particle counting
-// its partners) meets it: add(h, c) with c = 1, or 2 where both directions
-// share the index (equal types).  Where the lattice allows, the half stencil
-// meets each pair once and adds both directions, half the candidates.
-template <class F>
-__device__ __forceinline__ void rdf_pairs(const RdRep& R, const uint32_t* __restrict__ start,
-                                          const float4* __restrict__ ps, int s, float4 p, int nt, int S, float rmax,
-                                          float rcut2, int nbins, F&& add)
-{
-    const int ti = w_type(p.w);
-    int cx, cy, cz;
-    cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
-    const bool wrap = stencil_wraps(R, cx, cy, cz, S);
-    const bool half = 2 * S + 1 < R.L[0] && 2 * S + 1 < R.L[1] && 2 * S + 1 < R.L[2];
-    if (half) {
-        for_stencil_half_q(R, start, ps, (uint32_t)s, cx, cy, cz, S, [&](uint32_t j, float4 q) {
-            const int b = rdf_bin(R, p, q, rmax, rcut2, nbins, wrap);
-            if (b < 0) return;
-            const int tj = w_type(q.w);
-            const int h1 = (ti * nt + tj) * nbins + b, h2 = (tj * nt + ti) * nbins + b;
-            if (h1 == h2) {
-                add(h1, 2u);
-            } else {
-                add(h1, 1u);
-                add(h2, 1u);
-            }
-        });
-    } else {
-        for_stencil_q(R, start, ps, cx, cy, cz, S, [&](uint32_t j, float4 q) {
-            if ((int)j == s) return;
-            const int b = rdf_bin(R, p, q, rmax, rcut2, nbins, wrap);
-            if (b >= 0) add((ti * nt + w_type(q.w)) * nbins + b, 1u);
-        });
-    }
-}
-
-// One LDS histogram per workgroup, shared by its waves when their work items
-// belong to one replica (a workgroup straddling two replicas adds to the
-// global counts directly).  Workgroup b adds its histogram to copy b % ncopy
-// of the counts; k_rdf_fold sums the copies, so the 64-bit atomics of
-// thousands of workgroups do not queue on the same few thousand addresses.
-__global__ __launch_bounds__(RD_BLOCK) void k_rdf_lds(const float4* __restrict__ ps, const uint32_t* __restrict__ start,
-                                                      const RdDev* __restrict__ P, const RdRep* __restrict__ reps,
-                                                      const RdWave* __restrict__ waves, int nwaves, int S, float rmax,
-                                                      float rcut2, int nbins, unsigned long long* __restrict__ part,
-                                                      long part_stride, int ncopy,
-                                                      unsigned long long* __restrict__ counts)
-{
+    constexpr int ITEMS = BLOCK / G / 64;
+    static_assert(ITEMS >= 1 && ITEMS * 64 * G == BLOCK, "whole work items per workgroup");
     extern __shared__ uint32_t hist[];
-    __shared__ int rep_sh[RD_BLOCK / 64];
     const int nt = P->nt;
-    const int nh = nt * nt * nbins;
-    const RdWave it = wave_item(waves, nwaves, __builtin_amdgcn_readfirstlane(wave_id()));
-    if ((threadIdx.x & 63) == 0) rep_sh[threadIdx.x >> 6] = it.s1 > it.s0 ? it.rep : -1;
-    for (int k = threadIdx.x; k < nh; k += RD_BLOCK) hist[k] = 0u;
-    __syncthreads();
-    int rep0 = -1;
-    bool one = true;
-    for (int v = 0; v < RD_BLOCK / 64; ++v) {
-        const int r = rep_sh[v];
-        if (r < 0) continue;
-        if (rep0 < 0) rep0 = r;
-        else if (r != rep0) one = false;
-    }
-    const int s = it.s0 + (threadIdx.x & 63);
-    if (s < it.s1) {
-        const RdRep R = reps[it.rep];
-        unsigned long long* cnt = counts + (size_t)it.rep * nh;
-        const float4 p = ps[s];
-        rdf_pairs(R, start, ps, s, p, nt, S, rmax, rcut2, nbins, [&](int h, uint32_t c) {
-            if (one) atomicAdd(&hist[h], c);
-            else atomicAdd(&cnt[h], (unsigned long long)c);
-        });
-    }
-    __syncthreads();
-    if (one && rep0 >= 0) {
-        unsigned long long* cnt = part + (size_t)(blockIdx.x % ncopy) * (size_t)part_stride + (size_t)rep0 * nh;
-        for (int k = threadIdx.x; k < nh; k += RD_BLOCK) {
-            const uint32_t v = hist[k];
-            if (v) atomicAdd(&cnt[k], (unsigned long long)v);
+    const int nh = nt * nt * rdf.nbins;
+    const int w0 = xcd_block(blockIdx.x, gridDim.x) * ITEMS, w1 = min(nwaves, w0 + ITEMS);
+    const int lp = (int)threadIdx.x / G;             // particle of this lane in the workgroup
+    unsigned long long* copy = part + (size_t)(blockIdx.x % ncopy) * (size_t)part_stride;
+    for (int k = threadIdx.x; k < nh; k += BLOCK) hist[k] = 0u;
+    for (int w = w0; w < w1;) {
+        const int rep = waves[w].rep;
+        const int end = min(w1, waves[w].next);      // items of this replica in the share
+        __syncthreads();
+        const RdRep R = reps[rep];
+        const int i = __builtin_amdgcn_readfirstlane(w0 + lp / 64);
+        if (i >= w && i < end) {
+            const RdWave it = waves[i];
+            const int s = it.s0 + lp % 64;
+            if (s < it.s1) {
+                const float4 p = ps[s];
+                const int row = w_type(p.w) * nt * rdf.nbins;
+                for_pairs_once<G, W>(R, start, ps, (uint32_t)s, p, S, rdf.rmax, (int)threadIdx.x % G, [&](float4 q) {
+                    const int b = rdf_bin(rdf, set_dist2(R, p, q));
+                    if (b >= 0)
+                        atomicAdd(&hist[row + (int)__umul24((unsigned)w_type(q.w), (unsigned)rdf.nbins) + b], 1u);
+                });
+            }
         }
+        __syncthreads();
+        for (int k = threadIdx.x; k < nh; k += BLOCK) {
+            const uint32_t v = hist[k];
+            if (v) atomicAdd(&copy[(size_t)rep * nh + k], (unsigned long long)v);
+            if (end < w1) hist[k] = 0u;
+        }
+        w = end;
     }
 }
 
-// counts += the sum of the copies; the copies are cleared for the next call
-__global__ __launch_bounds__(RD_BLOCK) void k_rdf_fold(unsigned long long* __restrict__ part, long n, int ncopy,
-                                                       unsigned long long* __restrict__ counts)
+// counts(a, b) = the copies' pairs at (a, b) and at (b, a) (the copies hold
+// all frames so far)
+__global__ __launch_bounds__(RD_BLOCK) void k_rdf_fold(const unsigned long long* __restrict__ part, long n, int ncopy,
+                                                       int nt, int nbins, unsigned long long* __restrict__ counts)
 {
     const long i = (long)blockIdx.x * RD_BLOCK + threadIdx.x;
     if (i >= n) return;
+    const long bin = i % nbins, ab = i / nbins;
+    const long b = ab % nt, a = ab / nt % nt, rep = ab / ((long)nt * nt);
+    const long j = ((rep * nt + b) * nt + a) * nbins + bin;
     unsigned long long v = 0;
-    for (int c = 0; c < ncopy; ++c) {
-        v += part[(size_t)c * n + i];
-        part[(size_t)c * n + i] = 0ull;
-    }
-    counts[i] += v;
+    for (int c = 0; c < ncopy; ++c) v += part[(size_t)c * n + i] + part[(size_t)c * n + j];
+    counts[i] = v;
 }
 
-// histogram too large for LDS: direct 64-bit atomics on the global counts
+// histogram too large for LDS: direct 64-bit atomics on the global counts,
+// both orders of a pair
 __global__ __launch_bounds__(RD_BLOCK) void k_rdf_global(const float4* __restrict__ ps,
                                                          const uint32_t* __restrict__ start,
                                                          const RdDev* __restrict__ P, const RdRep* __restrict__ reps,
                                                          const RdWave* __restrict__ waves, int nwaves, int S,
-                                                         float rmax, float rcut2, int nbins,
-                                                         unsigned long long* __restrict__ counts)
+                                                         RdRdf rdf, unsigned long long* __restrict__ counts)
 {
-    const int nt = P->nt;
-    const int nh = nt * nt * nbins;
+    const int nt = P->nt, nbins = rdf.nbins;
+    const size_t nh = (size_t)nt * nt * nbins;
     const RdWave it = wave_item(waves, nwaves, wave_id());
     const int s = it.s0 + (threadIdx.x & 63);
     if (s >= it.s1) return;
     const RdRep R = reps[it.rep];
     unsigned long long* cnt = counts + (size_t)it.rep * nh;
     const float4 p = ps[s];
-    rdf_pairs(R, start, ps, s, p, nt, S, rmax, rcut2, nbins,
-              [&](int h, uint32_t c) { atomicAdd(&cnt[h], (unsigned long long)c); });
+    const int ti = w_type(p.w);
+    for_pairs_once<1, 2>(R, start, ps, (uint32_t)s, p, S, rdf.rmax, 0, [&](float4 q) {
+        const int b = rdf_bin(rdf, set_dist2(R, p, q));
+        if (b < 0) return;
+        const int tj = w_type(q.w);
+        atomicAdd(&cnt[(size_t)(ti * nt + tj) * nbins + b], 1ull);
+        atomicAdd(&cnt[(size_t)(tj * nt + ti) * nbins + b], 1ull);
+    });
 }
 
 // pairs (i<j by index) with d2 < thr2[ti][tj]; global particle indices
@@ -817,20 +794,11 @@ __global__ __launch_bounds__(RD_BLOCK) void k_pairs(const float4* __restrict__ p
     int cx, cy, cz;
     cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
     const uint32_t o = EMIT ? cnt_off[gi] : 0u;
-    const bool wrap = stencil_wraps(R, cx, cy, cz, S);
     uint32_t c = 0;
     for_stencil_q(R, start, ps, cx, cy, cz, S, [&](uint32_t j, float4 q) {
         uint32_t jj = w_index(q.w);
         if (jj <= ii) return;
-        float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-        if (wrap) {
-            dx = min_image(dx, R.Lb[0], R.half[0]);
-            dy = min_image(dy, R.Lb[1], R.half[1]);
-            dz = min_image(dz, R.Lb[2], R.half[2]);
-        }
-        float d2 = dx * dx;
-        d2 = d2 + dy * dy;
-        d2 = d2 + dz * dz;
+        const float d2 = set_dist2(R, p, q);
         if (d2 < thr2[ti * nt + w_type(q.w)]) {
             if (EMIT) {
                 // insertion into the sorted segment
@@ -1175,9 +1143,11 @@ static int build_tables(rd_system* h)
     std::vector<RdWave> wave_tab;
     for (size_t r = 0; r < rep_dev.size(); ++r) {
         const RdRep& R = rep_dev[r];
+        const int next = (int)wave_tab.size() + (R.n + 63) / 64;
         for (int s = 0; s < R.n; s += 64) {
             RdWave w;
-            w.rep = (int)r; w.s0 = R.off + s; w.s1 = R.off + std::min(R.n, s + 64); w.pad = 0;
+            w.rep = (int)r; w.s0 = R.off + s; w.s1 = R.off + std::min(R.n, s + 64);
+            w.next = next;
             wave_tab.push_back(w);
         }
     }
@@ -1883,6 +1853,36 @@ extern "C" int rd_rdf_reset(rd_system* h)
     return rd_rdf_configure(h, h->rdf_rmax, h->rdf_bins);
 }
 
+template <int BLOCK, int G, int W>
+static hipError_t launch_rdf_form(rd_system* h, int S, const RdRdf& rdf, size_t lds, long total)
+{
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute((const void*)k_rdf_lds<BLOCK, G, W>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    const int grid = std::max(1, nblk(h->nwaves, BLOCK / G / 64));
+    hipLaunchKernelGGL((k_rdf_lds<BLOCK, G, W>), dim3(grid), dim3(BLOCK), lds, h->stream, h->d_ps, h->d_start, h->d_P,
+                       h->d_reps, h->d_waves, h->nwaves, S, rdf, h->d_rdf_part, total, h->rdf_ncopy);
+    return hipSuccess;
+}
+
+// Lanes per particle and workgroup size: 16 lanes (1,024 threads, one work
+// item at a time) up to two work items per compute unit, 4 lanes (512) up to
+// 16, 2 lanes (256) beyond.  A particle's half stencil has 25 to 61 rows; few
+// particles leave the chip waiting for one lane's chain through them, many
+// pay for each lane's set-up and each workgroup's flush.  Whole call at 200
+// bins, 20 nm, 16 / 4 / 2 lanes (us): 10,000 particles 45 / 85 / 146 (one lane
+// through the uncut half stencil with two atomics a pair: 461), 50,000
+// 54 / 46 / 59 (132), 200,000 134 / 85 / 82 (152), 1M 555 / 284 / 227 (321),
+// 64 replicas of 911,000 particles 665 / 399 / 338 (620).
+static hipError_t launch_rdf(rd_system* h, int S, const RdRdf& rdf, size_t lds, long total)
+{
+    if (h->nwaves <= 2 * h->ncu) return launch_rdf_form<1024, 16, 4>(h, S, rdf, lds, total);
+    if (h->nwaves <= 16 * h->ncu) return launch_rdf_form<512, 4, 4>(h, S, rdf, lds, total);
+    return launch_rdf_form<256, 2, 2>(h, S, rdf, lds, total);
+}
+
 extern "C" int rd_rdf_calculate(rd_system* h)
 {
     if (!h) return RD_EINVAL;
@@ -1895,20 +1895,21 @@ extern "C" int rd_rdf_calculate(rd_system* h)
     // one histogram per workgroup of up to 160 KB
     size_t lds = nh * sizeof(uint32_t);
     const float rmax = (float)h->rdf_rmax;
-    const float rcut2 = (float)((double)rmax * (double)rmax * (1.0 + 1e-6));
+    RdRdf rdf;
+    rdf.rmax = rmax;
+    rdf.rcut2 = (float)((double)rmax * (double)rmax * (1.0 + 1e-6));
+    rdf.nbins = h->rdf_bins;
+    rdf.scale = (float)((double)h->rdf_bins / (double)rmax);
+    rdf.margin = 1e-6f * (float)h->rdf_bins;
     if (h->n > 0) {
-        if (lds + 64 <= 160 * 1024 && h->d_rdf_part) {          // + the static replica table
-            if (lds > 64 * 1024)
-                HIPCK(h, hipFuncSetAttribute((const void*)k_rdf_lds, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (lds + 64 <= 160 * 1024 && h->d_rdf_part) {
             const long total = (long)h->rdf_nrep * (long)nh;
-            hipLaunchKernelGGL(k_rdf_lds, dim3(wave_blocks(h)), dim3(RD_BLOCK), lds, h->stream, h->d_ps, h->d_start,
-                               h->d_P, h->d_reps, h->d_waves, h->nwaves, S, rmax, rcut2, h->rdf_bins, h->d_rdf_part,
-                               total, h->rdf_ncopy, h->d_rdf);
+            HIPCK(h, launch_rdf(h, S, rdf, lds, total));
             hipLaunchKernelGGL(k_rdf_fold, dim3(std::max(1, nblk(total, RD_BLOCK))), dim3(RD_BLOCK), 0, h->stream,
-                               h->d_rdf_part, total, h->rdf_ncopy, h->d_rdf);
+                               h->d_rdf_part, total, h->rdf_ncopy, h->nt, h->rdf_bins, h->d_rdf);
         } else {
             hipLaunchKernelGGL(k_rdf_global, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_start,
-                               h->d_P, h->d_reps, h->d_waves, h->nwaves, S, rmax, rcut2, h->rdf_bins, h->d_rdf);
+                               h->d_P, h->d_reps, h->d_waves, h->nwaves, S, rdf, h->d_rdf);
         }
         HIPCK(h, hipGetLastError());
     }
