@@ -1,8 +1,8 @@
 // rd_mlp.h -- BF16 MLP 3 -> 64 -> 64 -> 64 -> 3 (SiLU) on gfx950 MFMA.
 //
-// One wave evaluates 64 samples with v_mfma_f32_16x16x32_bf16 (FP32
-// accumulation).  Lane l = 16 g + j holds, for every sample tile tj (samples
-// 16 tj + j) and feature tile ti, the four features 16 ti + 4 g + r, r = 0..3:
+// A wave evaluates tiles of 16 samples with v_mfma_f32_16x16x32_bf16 (FP32
+// accumulation).  Lane l = 16 g + j holds, for sample j of the tile and every
+// feature tile ti, the four features 16 ti + 4 g + r, r = 0..3:
 // exactly the accumulator layout of the 16x16 MFMA (column j, rows 4g + r).
 // The same registers serve as the B operand of the next layer when the
 // weights' K order is permuted to match: logical k = 8 g + t of K-block kb is
@@ -75,109 +75,39 @@ __device__ __forceinline__ float rd_dsilu(float z)
     return s * (1.0f + z * (1.0f - s));
 }
 
-// B operand for sample tile tj, K-block kb, from the lane's activations
-__device__ __forceinline__ rd_bf16x8 rd_mlp_bop(const float (&a)[4][4][4], int tj, int kb)
+// B operand of K-block kb from the lane's activations of one sample tile
+__device__ __forceinline__ rd_bf16x8 rd_mlp_bop(const float (&a)[4][4], int kb)
 {
     rd_bf16x8 v;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) v[t] = (__bf16)a[tj][2 * kb + t / 4][t & 3];
+    for (int t = 0; t < 8; ++t) v[t] = (__bf16)a[2 * kb + t / 4][t & 3];
     return v;
 }
 
 #define RD_MFMA(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16((A), (B), (C), 0, 0, 0)
 
-// z = W h + b for a 64x64 layer; A(to, kb) returns the lane's weight fragment
-template <class AF>
-__device__ __forceinline__ void rd_mlp_layer64(AF&& A, const float* __restrict__ b, const float (&h)[4][4][4],
-                                               float (&z)[4][4][4], int lane)
+// z = W h + b of a 64x64 layer for one sample tile; w: the lane's weight
+// fragments, b: the lane's biases (features 16 to + 4 g + r), or 0
+__device__ __forceinline__ void rd_mlp_layer64(const rd_bf16x8 (&w)[4][2], const rd_f32x4 (&b)[4],
+                                               const float (&h)[4][4], float (&z)[4][4])
 {
-    rd_bf16x8 bop[4][2];
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-        bop[tj][0] = rd_mlp_bop(h, tj, 0);
-        bop[tj][1] = rd_mlp_bop(h, tj, 1);
-    }
-    const int g = lane >> 4;
+    const rd_bf16x8 h0 = rd_mlp_bop(h, 0), h1 = rd_mlp_bop(h, 1);
 #pragma unroll
     for (int to = 0; to < 4; ++to) {
-        const rd_bf16x8 a0 = A(to, 0), a1 = A(to, 1);
-        rd_f32x4 bias;
+        rd_f32x4 acc = b[to];
+        acc = RD_MFMA(w[to][0], h0, acc);
+        acc = RD_MFMA(w[to][1], h1, acc);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) bias[r] = b[to * 16 + 4 * g + r];
-#pragma unroll
-        for (int tj = 0; tj < 4; ++tj) {
-            rd_f32x4 acc = bias;
-            acc = RD_MFMA(a0, bop[tj][0], acc);
-            acc = RD_MFMA(a1, bop[tj][1], acc);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) z[tj][to][r] = acc[r];
-        }
+        for (int r = 0; r < 4; ++r) z[to][r] = acc[r];
     }
 }
 
-// layer 1 on the VALU: z1 = W1 xn + b1 for the lane's 4 samples
-__device__ __forceinline__ void rd_mlp_layer1(const float* __restrict__ w1, const float* __restrict__ b1,
-                                              const float (&xn)[4][3], float (&z)[4][4][4], int lane)
-{
-    const int g = lane >> 4;
-#pragma unroll
-    for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int f = ti * 16 + 4 * g + r;
-            const float wa = w1[3 * f], wb = w1[3 * f + 1], wc = w1[3 * f + 2], bb = b1[f];
-#pragma unroll
-            for (int tj = 0; tj < 4; ++tj) {
-                float v = wa * xn[tj][0];
-                v = v + wb * xn[tj][1];
-                v = v + wc * xn[tj][2];
-                z[tj][ti][r] = v + bb;
-            }
-        }
-}
-
-// layer 4: y[tj][0..2] valid in lanes 0..15 (sample 16 tj + lane); A(kb)
-// returns the lane's fragment of W4 (rows 3..15 zero)
-template <class AF>
-__device__ __forceinline__ void rd_mlp_layer4(AF&& A, const float* __restrict__ b4, const float (&h)[4][4][4],
-                                              float (&y)[4][3], int lane)
-{
-    const rd_bf16x8 a0 = A(0), a1 = A(1);
-    const int g = lane >> 4;
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-        rd_f32x4 acc;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] = (g == 0 && r < 3) ? b4[r] : 0.0f;
-        acc = RD_MFMA(a0, rd_mlp_bop(h, tj, 0), acc);
-        acc = RD_MFMA(a1, rd_mlp_bop(h, tj, 1), acc);
-        y[tj][0] = acc[0]; y[tj][1] = acc[1]; y[tj][2] = acc[2];
-    }
-}
-
-__device__ __forceinline__ void rd_mlp_silu_all(const float (&z)[4][4][4], float (&h)[4][4][4])
+__device__ __forceinline__ void rd_mlp_silu_all(const float (&z)[4][4], float (&h)[4][4])
 {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) h[a][b][r] = rd_silu(z[a][b][r]);
-}
-
-// Move the outputs so that lane l holds sample l (y[tj] of lane l%16 for tj = l/16).
-__device__ __forceinline__ float3 rd_mlp_gather_out(const float (&y)[4][3], int lane)
-{
-    const int src = lane & 15, tj = lane >> 4;
-    float o[3] = { 0.0f, 0.0f, 0.0f };
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            float v = __shfl(y[t][c], src, 64);
-            if (t == tj) o[c] = v;
-        }
-    return make_float3(o[0], o[1], o[2]);
+        for (int r = 0; r < 4; ++r) h[b][r] = rd_silu(z[b][r]);
 }
 
 // sum over the 16 lanes of a lane group (lanes with equal lane>>4)

@@ -239,26 +239,42 @@ __global__ __launch_bounds__(256) void k_sur_normalise(float4* __restrict__ tg, 
 }
 
 // ===========================================================================
-// Training: forward + backward per wave of 64 samples -> partial gradients
+// Training: forward + backward of 64 samples per workgroup -> partial gradients
 // ===========================================================================
 struct RdTrainCtl {
     unsigned long long step;   // optimiser steps taken
+    unsigned long long cur;    // the step being taken (written by k_mlp_train for k_mlp_adam)
     float loss;                // loss of the last step
-    float pad;
+    float lr, c1, c2;          // its learning rate and bias corrections
 };
 
-#define RD_TLD 72   // row stride (bf16) of the per-wave staging matrices [64][RD_TLD]
+#define RD_TLD 72   // row stride (bf16) of the staging matrices [64][RD_TLD]
+#define RD_TLF 68   // row stride (float) of the FP32 one: 4 rows apart is 16 banks apart
 
-// activations (C layout) -> staging matrix S[feature][sample] in BF16
-__device__ __forceinline__ void stage_act(__bf16* S, const float (&a)[4][4][4], int lane)
+// one stage of the backward pass, shared by the workgroup's waves: dz and the
+// layer's input in BF16 ([feature][sample]), dz in FP32
+struct RdTrainStage {
+    __bf16 d[64 * RD_TLD], h[64 * RD_TLD];
+    float f[64 * RD_TLF];
+};
+
+// the wave's sample columns (tile wv) of a stage
+__device__ __forceinline__ void stage_bf16(__bf16* S, const float (&a)[4][4], int wv, int lane)
 {
     const int j = lane & 15, g = lane >> 4;
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
+    for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
-        for (int ti = 0; ti < 4; ++ti)
+        for (int r = 0; r < 4; ++r) S[(ti * 16 + 4 * g + r) * RD_TLD + wv * 16 + j] = (__bf16)a[ti][r];
+}
+
+__device__ __forceinline__ void stage_f32(float* S, const float (&a)[4][4], int wv, int lane)
+{
+    const int j = lane & 15, g = lane >> 4;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) S[(ti * 16 + 4 * g + r) * RD_TLD + tj * 16 + j] = (__bf16)a[tj][ti][r];
+    for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[(ti * 16 + 4 * g + r) * RD_TLF + wv * 16 + j] = a[ti][r];
 }
 
 __device__ __forceinline__ rd_bf16x8 lds_frag(const __bf16* S, int row, int col)
@@ -266,136 +282,175 @@ __device__ __forceinline__ rd_bf16x8 lds_frag(const __bf16* S, int row, int col)
     return *reinterpret_cast<const rd_bf16x8*>(S + row * RD_TLD + col);
 }
 
-// dW[i][k] = sum_samples D[i][s] H[k][s] for 64x64, written to out (row-major [64][64])
-__device__ __forceinline__ void wgrad64(const __bf16* SD, const __bf16* SH, float* __restrict__ out, int lane)
+// rows 16 ti .. 16 ti + 15 of dW[i][k] = sum_samples D[i][s] H[k][s] (64x64),
+// written to out (row-major [64][64])
+__device__ __forceinline__ void wgrad_rows(const RdTrainStage& S, int ti, float* __restrict__ out, int lane)
 {
     const int j = lane & 15, g = lane >> 4;
+    const rd_bf16x8 a0 = lds_frag(S.d, ti * 16 + j, 8 * g), a1 = lds_frag(S.d, ti * 16 + j, 32 + 8 * g);
+#pragma unroll
+    for (int tk = 0; tk < 4; ++tk) {
+        rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
+        acc = RD_MFMA(a0, lds_frag(S.h, tk * 16 + j, 8 * g), acc);
+        acc = RD_MFMA(a1, lds_frag(S.h, tk * 16 + j, 32 + 8 * g), acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[(ti * 16 + 4 * g + r) * 64 + tk * 16 + j] = acc[r];
+    }
+}
+
+// bias gradient of features 16 ti .. 16 ti + 15: sum over the 64 samples of dz
+__device__ __forceinline__ void bgrad_rows(const RdTrainStage& S, int ti, float* __restrict__ out, int lane)
+{
+    const int j = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float* d = S.f + (ti * 16 + 4 * g + r) * RD_TLF + j;
+        const float v = rd_sum16(d[0] + d[16] + d[32] + d[48]);
+        if (j == 0) out[ti * 16 + 4 * g + r] = v;
+    }
+}
+
+// dz of the layer below: (W^T dz) dsilu(z), W^T fragments wt
+__device__ __forceinline__ void back64(const rd_bf16x8 (&wt)[4][2], const float (&z)[4][4], float (&dz)[4][4])
+{
+    const rd_f32x4 zero[4] = {};
+    float dh[4][4];
+    rd_mlp_layer64(wt, zero, dz, dh);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dz[b][r] = dh[b][r] * rd_dsilu(z[b][r]);
+}
+
+// Learning rate (cosine from lr0 to lr1 over total steps) and Adam's bias
+// corrections.
+struct RdSchedule {
+    float lr0, lr1;
+    long long total;
+    float b1, b2;
+};
+
+// Samples: idx = sequential ? c : Philox(seed, step, c) mod m.  Samples at
+// c >= batch (padding of the last workgroup) contribute nothing.
+//
+// A batch is small for the chip (8,192 samples: 128 workgroups of 64), so the
+// step is bound by its chain of latencies: each of the four waves takes 16
+// samples through the network and back, all weight fragments are loaded to
+// registers up front, and the waves meet once per layer, at a stage in LDS
+// (two, used in turn, so that one barrier per stage suffices) from which each
+// wave computes a quarter of the layer's weight and bias gradients.  256
+// steps of 8,192 samples with k_mlp_adam: FIG us a step, against 55 us with
+// 64 samples in each wave (32 workgroups), weights staged in LDS and the step
+// counter in a kernel of its own.  The sums' orders are those of that form.
+// One more workgroup computes the step's schedule meanwhile.
+__global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn_all, const float4* __restrict__ tn_all,
+                                                   long m, int batch, int sequential, uint64_t seed,
+                                                   const RdMlpPack* __restrict__ pk, RdTrainCtl* __restrict__ ctl,
+                                                   float* __restrict__ partial, RdSchedule sch)
+{
+    __shared__ __align__(16) RdTrainStage stage[2];
+    __shared__ float xs[3][64], rs[3][64];           // inputs and residuals of the samples
+    const unsigned long long step = ctl->step;
+    if (blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x == 0) {
+            const unsigned long long t = step + 1;
+            const double ph = sch.total > 0 ? fmin(1.0, (double)(t - 1) / (double)sch.total) : 0.0;
+            ctl->cur = step;
+            ctl->lr = sch.lr1 + 0.5f * (sch.lr0 - sch.lr1) * (float)(1.0 + cos(3.14159265358979323846 * ph));
+            ctl->c1 = 1.0f - (float)pow((double)sch.b1, (double)t);
+            ctl->c2 = 1.0f - (float)pow((double)sch.b2, (double)t);
+        }
+        return;
+    }
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int j = lane & 15, g = lane >> 4;
+    float* out = partial + (size_t)blockIdx.x * RD_MLP_ROW;
+
+    const int c = blockIdx.x * 64 + wv * 16 + j;
+    const bool live = c < batch;
+    long idx = c;
+    if (!sequential) {
+        uint32_t q[4] = { (uint32_t)c, (uint32_t)step, (uint32_t)(step >> 32), 0x5452414eu };
+        philox4x32_10(q, (uint32_t)seed, (uint32_t)(seed >> 32));
+        idx = (long)(((uint64_t)q[1] << 32 | q[0]) % (uint64_t)m);
+    }
+    if (!live) idx = 0;
+    const float4 xa = xn_all[idx], ta = tn_all[idx];
+    // the lane's weights: layer 1 (features 16 ti + 4 g + r: 12 consecutive
+    // values per tile), biases, and the fragments of every layer
+    rd_f32x4 w1[4][3], b1[4], b2[4], b3[4];
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti) {
-        rd_bf16x8 a0 = lds_frag(SD, ti * 16 + j, 8 * g), a1 = lds_frag(SD, ti * 16 + j, 32 + 8 * g);
+        const int f = ti * 16 + 4 * g;
+        b1[ti] = *reinterpret_cast<const rd_f32x4*>(pk->b1 + f);
+        b2[ti] = *reinterpret_cast<const rd_f32x4*>(pk->b2 + f);
+        b3[ti] = *reinterpret_cast<const rd_f32x4*>(pk->b3 + f);
 #pragma unroll
-        for (int tk = 0; tk < 4; ++tk) {
-            rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-            acc = RD_MFMA(a0, lds_frag(SH, tk * 16 + j, 8 * g), acc);
-            acc = RD_MFMA(a1, lds_frag(SH, tk * 16 + j, 32 + 8 * g), acc);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) out[(ti * 16 + 4 * g + r) * 64 + tk * 16 + j] = acc[r];
-        }
+        for (int k = 0; k < 3; ++k) w1[ti][k] = *reinterpret_cast<const rd_f32x4*>(pk->w1 + 3 * f + 4 * k);
     }
-}
+    rd_bf16x8 w2[4][2], w3[4][2], w2t[4][2], w3t[4][2], w4[2], w4t[4];
+#pragma unroll
+    for (int to = 0; to < 4; ++to)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) w2[to][kb] = pk->w2[to][kb][lane];
+#pragma unroll
+    for (int to = 0; to < 4; ++to)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) w3[to][kb] = pk->w3[to][kb][lane];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) w4[kb] = pk->w4[kb][lane];
+#pragma unroll
+    for (int to = 0; to < 4; ++to) w4t[to] = pk->w4t[to][lane];
+#pragma unroll
+    for (int to = 0; to < 4; ++to)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) w3t[to][kb] = pk->w3t[to][kb][lane];
+#pragma unroll
+    for (int to = 0; to < 4; ++to)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) w2t[to][kb] = pk->w2t[to][kb][lane];
+    rd_f32x4 b4 = { 0.f, 0.f, 0.f, 0.f };
+    if (g == 0) { b4[0] = pk->b4[0]; b4[1] = pk->b4[1]; b4[2] = pk->b4[2]; }
+    const float xn[3] = { xa.x, xa.y, xa.z }, tn[3] = { ta.x, ta.y, ta.z };
 
-// dH = W^T dZ with W^T fragments wt[to][kb][lane]; dZ in the C layout
-template <class WP>
-__device__ __forceinline__ void back64(const WP& wt, const float (&dz)[4][4][4], float (&dh)[4][4][4], int lane)
-{
-    rd_bf16x8 bop[4][2];
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-        bop[tj][0] = rd_mlp_bop(dz, tj, 0);
-        bop[tj][1] = rd_mlp_bop(dz, tj, 1);
-    }
-#pragma unroll
-    for (int to = 0; to < 4; ++to) {
-        const rd_bf16x8 a0 = wt[to][0][lane], a1 = wt[to][1][lane];
-#pragma unroll
-        for (int tj = 0; tj < 4; ++tj) {
-            rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-            acc = RD_MFMA(a0, bop[tj][0], acc);
-            acc = RD_MFMA(a1, bop[tj][1], acc);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dh[tj][to][r] = acc[r];
-        }
-    }
-}
-
-// bias gradient: sum over the 64 samples of d[.][ti][r]; lanes j == 0 write
-__device__ __forceinline__ void bgrad(const float (&d)[4][4][4], float* __restrict__ out, int lane)
-{
-    const int j = lane & 15, g = lane >> 4;
+    // ---- forward ----
+    float z1[4][4], z2[4][4], z3[4][4], h[4][4];
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            float v = d[0][ti][r] + d[1][ti][r] + d[2][ti][r] + d[3][ti][r];
-            v = rd_sum16(v);
-            if (j == 0) out[ti * 16 + 4 * g + r] = v;
+            const int k = 3 * r;
+            float v = w1[ti][k / 4][k % 4] * xn[0];
+            v = v + w1[ti][(k + 1) / 4][(k + 1) % 4] * xn[1];
+            v = v + w1[ti][(k + 2) / 4][(k + 2) % 4] * xn[2];
+            z1[ti][r] = v + b1[ti][r];
         }
-}
-
-// Samples: idx = sequential ? c : Philox(seed, step, c) mod m.  Samples at
-// c >= batch (padding of the last wave) contribute nothing.
-__global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn_all, const float4* __restrict__ tn_all,
-                                                   long m, int batch, int sequential, uint64_t seed,
-                                                   const RdMlpPack* __restrict__ pk_g, RdTrainCtl* __restrict__ ctl,
-                                                   float* __restrict__ partial)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    RdMlpPack& pk = *reinterpret_cast<RdMlpPack*>(smem);
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    __bf16* SD = reinterpret_cast<__bf16*>(smem + sizeof(RdMlpPack)) + (size_t)wv * 2 * 64 * RD_TLD;
-    __bf16* SH = SD + 64 * RD_TLD;
-    {
-        const uint4* src = reinterpret_cast<const uint4*>(pk_g);
-        uint4* dst = reinterpret_cast<uint4*>(smem);
-        for (int i = threadIdx.x; i < (int)(sizeof(RdMlpPack) / 16); i += 256) dst[i] = src[i];
-    }
-    __syncthreads();
-    const unsigned long long step = ctl->step;
-    const int w = blockIdx.x * 4 + wv;
-    const int j = lane & 15, g = lane >> 4;
-    float* out = partial + (size_t)w * RD_MLP_ROW;
-
-    float xn[4][3], tn[4][3];
-    bool live[4];
-#pragma unroll
-    for (int tj = 0; tj < 4; ++tj) {
-        const int c = w * 64 + tj * 16 + j;
-        live[tj] = c < batch;
-        long idx = c;
-        if (!sequential) {
-            uint32_t q[4] = { (uint32_t)c, (uint32_t)step, (uint32_t)(step >> 32), 0x5452414eu };
-            philox4x32_10(q, (uint32_t)seed, (uint32_t)(seed >> 32));
-            idx = (long)(((uint64_t)q[1] << 32 | q[0]) % (uint64_t)m);
-        }
-        if (!live[tj]) idx = 0;
-        float4 a = xn_all[idx], b = tn_all[idx];
-        xn[tj][0] = a.x; xn[tj][1] = a.y; xn[tj][2] = a.z;
-        tn[tj][0] = b.x; tn[tj][1] = b.y; tn[tj][2] = b.z;
-    }
-
-    // ---- forward ----
-    float z1[4][4][4], z2[4][4][4], z3[4][4][4], h[4][4][4];
-    rd_mlp_layer1(pk.w1, pk.b1, xn, z1, lane);
     rd_mlp_silu_all(z1, h);
-    rd_mlp_layer64([&](int to, int kb) { return pk.w2[to][kb][lane]; }, pk.b2, h, z2, lane);
+    rd_mlp_layer64(w2, b2, h, z2);
     rd_mlp_silu_all(z2, h);
-    rd_mlp_layer64([&](int to, int kb) { return pk.w3[to][kb][lane]; }, pk.b3, h, z3, lane);
+    rd_mlp_layer64(w3, b3, h, z3);
     rd_mlp_silu_all(z3, h);                  // h = h3
-    float y[4][3];
-    rd_mlp_layer4([&](int kb) { return pk.w4[kb][lane]; }, pk.b4, h, y, lane);
+    rd_f32x4 y = b4;
+    y = RD_MFMA(w4[0], rd_mlp_bop(h, 0), y);
+    y = RD_MFMA(w4[1], rd_mlp_bop(h, 1), y);
 
-    // ---- loss and dy (lanes of group 0 hold the outputs) ----
+    // ---- residuals and dy (lanes of group 0 hold the outputs) ----
     const float sc2 = 2.0f / (float)batch;
-    float dy[4][3];
-    float lsum = 0.0f;
+    float dy[3];
+    __bf16* const SD = stage[0].d;
+    stage_bf16(stage[0].h, h, wv, lane);
 #pragma unroll
-    for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            float r = (g == 0 && live[tj]) ? y[tj][c] - tn[tj][c] : 0.0f;
-            lsum += r * r;
-            dy[tj][c] = sc2 * r;
+    for (int k = 0; k < 3; ++k) {
+        const float r = (g == 0 && live) ? y[k] - tn[k] : 0.0f;
+        dy[k] = sc2 * r;
+        if (g == 0) {
+            SD[k * RD_TLD + wv * 16 + j] = (__bf16)dy[k];
+            rs[k][wv * 16 + j] = r;
+            xs[k][wv * 16 + j] = xn[k];
         }
-
-    // dW4 = dy h3^T: stage dy (rows 0..2) and h3
-    stage_act(SH, h, lane);
-    if (g == 0) {
-#pragma unroll
-        for (int tj = 0; tj < 4; ++tj)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) SD[c * RD_TLD + tj * 16 + j] = (__bf16)dy[tj][c];
     }
     __syncthreads();
+    // columns 16 wv .. of dW4 = dy h3^T
     {
         rd_bf16x8 a0, a1;
         if (j < 3) { a0 = lds_frag(SD, j, 8 * g); a1 = lds_frag(SD, j, 32 + 8 * g); }
@@ -403,103 +458,86 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn
 #pragma unroll
             for (int t = 0; t < 8; ++t) { a0[t] = (__bf16)0.0f; a1[t] = (__bf16)0.0f; }
         }
+        rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
+        acc = RD_MFMA(a0, lds_frag(stage[0].h, wv * 16 + j, 8 * g), acc);
+        acc = RD_MFMA(a1, lds_frag(stage[0].h, wv * 16 + j, 32 + 8 * g), acc);
+        if (g == 0) {
 #pragma unroll
-        for (int tk = 0; tk < 4; ++tk) {
-            rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-            acc = RD_MFMA(a0, lds_frag(SH, tk * 16 + j, 8 * g), acc);
-            acc = RD_MFMA(a1, lds_frag(SH, tk * 16 + j, 32 + 8 * g), acc);
-            if (g == 0) {
-#pragma unroll
-                for (int r = 0; r < 3; ++r) out[RD_MLP_W4 + r * 64 + tk * 16 + j] = acc[r];
-            }
+            for (int r = 0; r < 3; ++r) out[RD_MLP_W4 + r * 64 + wv * 16 + j] = acc[r];
         }
     }
     // db4 and the loss
+    if (wv == 0) {
+        float l = 0.0f, d4[3] = { 0.0f, 0.0f, 0.0f };
+        if (g == 0) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        float v = rd_sum16(dy[0][c] + dy[1][c] + dy[2][c] + dy[3][c]);
-        if (lane == 0) out[RD_MLP_B4 + c] = v;
-    }
-    {
-        float l = lsum;
+            for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float r = rs[k][tj * 16 + j];
+                    l += r * r;
+                    d4[k] = tj == 0 ? sc2 * r : d4[k] + sc2 * r;
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float v = rd_sum16(d4[k]);
+            if (lane == 0) out[RD_MLP_B4 + k] = v;
+        }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
         if (lane == 0) out[RD_MLP_NPARAM] = l / (float)batch;
     }
 
-    // dh3 = W4^T dy: B operand = dy in lanes of group 0 (k = 0..2)
-    float dz[4][4][4], dh[4][4][4];
+    // dz3 = (W4^T dy) dsilu: B operand = dy in lanes of group 0 (k = 0..2)
+    float dz[4][4];
     {
+        rd_bf16x8 b;
 #pragma unroll
-        for (int tj = 0; tj < 4; ++tj) {
-            rd_bf16x8 b;
+        for (int t = 0; t < 8; ++t) b[t] = (__bf16)((g == 0 && t < 3) ? dy[t < 3 ? t : 0] : 0.0f);
 #pragma unroll
-            for (int t = 0; t < 8; ++t) b[t] = (__bf16)((g == 0 && t < 3) ? dy[tj][t < 3 ? t : 0] : 0.0f);
+        for (int to = 0; to < 4; ++to) {
+            rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
+            acc = RD_MFMA(w4t[to], b, acc);
 #pragma unroll
-            for (int to = 0; to < 4; ++to) {
-                rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
-                acc = RD_MFMA(pk.w4t[to][lane], b, acc);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dh[tj][to][r] = acc[r];
-            }
+            for (int r = 0; r < 4; ++r) dz[to][r] = acc[r] * rd_dsilu(z3[to][r]);
         }
     }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dz[a][b][r] = dh[a][b][r] * rd_dsilu(z3[a][b][r]);
-    bgrad(dz, out + RD_MLP_B3, lane);
-
     // dW3 = dz3 h2^T
+    rd_mlp_silu_all(z2, h);
+    stage_bf16(stage[1].d, dz, wv, lane);
+    stage_bf16(stage[1].h, h, wv, lane);
+    stage_f32(stage[1].f, dz, wv, lane);
     __syncthreads();
-    rd_mlp_silu_all(z2, h);                  // h = h2
-    stage_act(SD, dz, lane);
-    stage_act(SH, h, lane);
-    __syncthreads();
-    wgrad64(SD, SH, out + RD_MLP_W3, lane);
-
-    // dh2 = W3^T dz3, dz2
-    back64(pk.w3t, dz, dh, lane);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dz[a][b][r] = dh[a][b][r] * rd_dsilu(z2[a][b][r]);
-    bgrad(dz, out + RD_MLP_B2, lane);
-
+    back64(w3t, z2, dz);                     // dz2
+    wgrad_rows(stage[1], wv, out + RD_MLP_W3, lane);
+    bgrad_rows(stage[1], wv, out + RD_MLP_B3, lane);
     // dW2 = dz2 h1^T
+    rd_mlp_silu_all(z1, h);
+    stage_bf16(stage[0].d, dz, wv, lane);
+    stage_bf16(stage[0].h, h, wv, lane);
+    stage_f32(stage[0].f, dz, wv, lane);
     __syncthreads();
-    rd_mlp_silu_all(z1, h);                  // h = h1
-    stage_act(SD, dz, lane);
-    stage_act(SH, h, lane);
+    back64(w2t, z1, dz);                     // dz1
+    wgrad_rows(stage[0], wv, out + RD_MLP_W2, lane);
+    bgrad_rows(stage[0], wv, out + RD_MLP_B2, lane);
+    // dW1 = dz1 xn^T in FP32 on the VALU
+    stage_f32(stage[1].f, dz, wv, lane);
     __syncthreads();
-    wgrad64(SD, SH, out + RD_MLP_W2, lane);
-
-    // dh1 = W2^T dz2, dz1 (FP32), dW1 = dz1 xn^T on the VALU
-    back64(pk.w2t, dz, dh, lane);
+    bgrad_rows(stage[1], wv, out + RD_MLP_B1, lane);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int r = 0; r < 4; ++r) {
+        const float* d = stage[1].f + (wv * 16 + 4 * g + r) * RD_TLF + j;
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dz[a][b][r] = dh[a][b][r] * rd_dsilu(z1[a][b][r]);
-    bgrad(dz, out + RD_MLP_B1, lane);
-#pragma unroll
-    for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                float v = dz[0][ti][r] * xn[0][c];
-                v = v + dz[1][ti][r] * xn[1][c];
-                v = v + dz[2][ti][r] * xn[2][c];
-                v = v + dz[3][ti][r] * xn[3][c];
-                v = rd_sum16(v);
-                if (j == 0) out[RD_MLP_W1 + 3 * (ti * 16 + 4 * g + r) + c] = v;
-            }
+        for (int k = 0; k < 3; ++k) {
+            float v = d[0] * xs[k][j];
+            v = v + d[16] * xs[k][16 + j];
+            v = v + d[32] * xs[k][32 + j];
+            v = v + d[48] * xs[k][48 + j];
+            v = rd_sum16(v);
+            if (j == 0) out[RD_MLP_W1 + 3 * (wv * 16 + 4 * g + r) + k] = v;
+        }
+    }
 }
 
 // write the packed BF16 / FP32 copies of master parameter p
@@ -561,26 +599,40 @@ __global__ __launch_bounds__(256) void k_mlp_pack(const float* __restrict__ mast
     if (p < RD_MLP_NPARAM) pack_param(pk, p, master[p]);
 }
 
-// Sum the partial gradients in wave order (deterministic), Adam step on the
-// FP32 master weights, refresh the packed copies.  Cosine learning rate from
-// lr0 to lr1 over total steps.
-__global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ partial, int nw,
+// Sum the partial gradients in row order (deterministic), Adam step on the
+// FP32 master weights, refresh the packed copies; the loss column's thread
+// advances the step counter (k_mlp_train reads it, nothing here does).
+__global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ partial, int nrow,
                                                   float* __restrict__ master, float* __restrict__ mom,
                                                   float* __restrict__ vel, RdMlpPack* __restrict__ pk,
-                                                  RdTrainCtl* __restrict__ ctl, float lr0, float lr1,
-                                                  long long total, float b1, float b2, float eps,
+                                                  RdTrainCtl* __restrict__ ctl, float b1, float b2, float eps,
                                                   float* __restrict__ grad_out, int apply,
                                                   float* __restrict__ loss_hist)
 {
-    // 32 parameters per workgroup, the per-wave partial rows split over 8
-    // slices, the slices added in a fixed order: deterministic, and enough
-    // workgroups to keep the loads in flight
+    // 32 parameters per workgroup, the partial rows split over 8 slices, the
+    // slices added in a fixed order: deterministic, and enough workgroups to
+    // keep the loads in flight (8 per thread at once)
     __shared__ float red[8][32];
     const int pl = threadIdx.x & 31, slice = threadIdx.x >> 5;
     const int p = blockIdx.x * 32 + pl;
+    const bool sum = slice == 0 && p < RD_MLP_NPARAM;
+    float m = 0.0f, v = 0.0f, w0 = 0.0f;
+    if (sum && apply) { m = mom[p]; v = vel[p]; w0 = master[p]; }
+    const unsigned long long cur = ctl->cur;
+    const float lr = ctl->lr, c1 = ctl->c1, c2 = ctl->c2;
     float part = 0.0f;
-    if (p <= RD_MLP_NPARAM)
-        for (int w = slice; w < nw; w += 8) part += partial[(size_t)w * RD_MLP_ROW + p];
+    if (p <= RD_MLP_NPARAM) {
+        const float* src = partial + p;
+        int w = slice;
+        for (; w + 56 < nrow; w += 64) {
+            float q[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) q[k] = src[(size_t)(w + 8 * k) * RD_MLP_ROW];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) part += q[k];
+        }
+        for (; w < nrow; w += 8) part += src[(size_t)w * RD_MLP_ROW];
+    }
     red[slice][pl] = part;
     __syncthreads();
     if (slice != 0 || p > RD_MLP_NPARAM) return;
@@ -589,26 +641,22 @@ __global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ part
     for (int k = 0; k < 8; ++k) gsum += red[k][pl];
     if (p == RD_MLP_NPARAM) {        // loss column
         ctl->loss = gsum;
-        if (loss_hist) loss_hist[ctl->step] = gsum;
+        if (loss_hist) loss_hist[cur] = gsum;
+        if (apply) ctl->step = cur + 1;
         return;
     }
     if (grad_out) grad_out[p] = gsum;
     if (!apply) return;
-    const unsigned long long t = ctl->step + 1;
-    const double ph = total > 0 ? fmin(1.0, (double)(t - 1) / (double)total) : 0.0;
-    const float lr = lr1 + 0.5f * (lr0 - lr1) * (float)(1.0 + cos(3.14159265358979323846 * ph));
-    float m = b1 * mom[p] + (1.0f - b1) * gsum;
-    float v = b2 * vel[p] + (1.0f - b2) * gsum * gsum;
+    m = b1 * m + (1.0f - b1) * gsum;
+    v = b2 * v + (1.0f - b2) * gsum * gsum;
     mom[p] = m;
     vel[p] = v;
-    const float mh = m / (1.0f - (float)pow((double)b1, (double)t));
-    const float vh = v / (1.0f - (float)pow((double)b2, (double)t));
-    const float w = master[p] - lr * mh / (sqrtf(vh) + eps);
+    const float mh = m / c1;
+    const float vh = v / c2;
+    const float w = w0 - lr * mh / (sqrtf(vh) + eps);
     master[p] = w;
     pack_param(pk, p, w);
 }
-
-__global__ void k_mlp_step_inc(RdTrainCtl* ctl) { ctl->step += 1; }
 
 // ===========================================================================
 // Inference
@@ -1110,22 +1158,14 @@ extern "C" int rd_surrogate_make_data(rd_system* h, long m, uint64_t seed, doubl
     return RD_OK;
 }
 
-static size_t train_lds() { return sizeof(RdMlpPack) + (size_t)4 * 2 * 64 * RD_TLD * sizeof(__bf16); }
-
 static int ensure_partial(rd_system* h, int batch)
 {
-    size_t rows = (size_t)((batch + 255) / 256) * 4;
+    const size_t rows = ((size_t)batch + 63) / 64;
     if (rows > h->partial_rows) {
         if (h->d_partial) (void)hipFree(h->d_partial);
         h->d_partial = nullptr;
         SHIPCK(h, hipMalloc(&h->d_partial, sizeof(float) * RD_MLP_ROW * rows));
         h->partial_rows = rows;
-    }
-    static bool attr = false;
-    if (!attr) {
-        SHIPCK(h, hipFuncSetAttribute((const void*)k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)train_lds()));
-        attr = true;
     }
     return RD_OK;
 }
@@ -1133,13 +1173,13 @@ static int ensure_partial(rd_system* h, int batch)
 static void launch_train_step(rd_system* h, const float4* xn, const float4* tn, long m, int batch, int sequential,
                               uint64_t seed, const rd_train_params& tp, float* grad_out, int apply, float* loss_hist)
 {
-    const int blocks = (batch + 255) / 256;
-    hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(256), train_lds(), h->stream, xn, tn, m, batch, sequential,
-                       seed, (const RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, h->d_partial);
-    hipLaunchKernelGGL(k_mlp_adam, dim3((RD_MLP_NPARAM + 1 + 31) / 32), dim3(256), 0, h->stream, h->d_partial, blocks * 4,
-                       h->d_master, h->d_mom, h->d_vel, (RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, tp.lr, tp.lr_min,
-                       (long long)tp.steps, tp.beta1, tp.beta2, tp.eps, grad_out, apply, loss_hist);
-    if (apply) hipLaunchKernelGGL(k_mlp_step_inc, dim3(1), dim3(1), 0, h->stream, (RdTrainCtl*)h->d_ctl);
+    const int rows = (batch + 63) / 64;
+    const RdSchedule sch = { tp.lr, tp.lr_min, (long long)tp.steps, tp.beta1, tp.beta2 };
+    hipLaunchKernelGGL(k_mlp_train, dim3(rows + 1), dim3(256), 0, h->stream, xn, tn, m, batch, sequential, seed,
+                       (const RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, h->d_partial, sch);
+    hipLaunchKernelGGL(k_mlp_adam, dim3((RD_MLP_NPARAM + 1 + 31) / 32), dim3(256), 0, h->stream, h->d_partial, rows,
+                       h->d_master, h->d_mom, h->d_vel, (RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, tp.beta1,
+                       tp.beta2, tp.eps, grad_out, apply, loss_hist);
 }
 
 // loss and gradient of one batch (no update): the gradient check entry
