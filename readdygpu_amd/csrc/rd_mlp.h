@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define RD_MLP_NPARAM 8771
 #define RD_MLP_W1 0
 #define RD_MLP_B1 192
@@ -68,12 +70,8 @@ __device__ __forceinline__ float rd_sigmoid(float z)
 {
     return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504f));
 }
-__device__ __forceinline__ float rd_silu(float z) { return z * rd_sigmoid(z); }
-__device__ __forceinline__ float rd_dsilu(float z)
-{
-    const float s = rd_sigmoid(z);
-    return s * (1.0f + z * (1.0f - s));
-}
+// derivative of SiLU from z and its sigmoid s
+__device__ __forceinline__ float rd_dsilu(float z, float s) { return s * (1.0f + z * (1.0f - s)); }
 
 // B operand of K-block kb from the lane's activations of one sample tile
 __device__ __forceinline__ rd_bf16x8 rd_mlp_bop(const float (&a)[4][4], int kb)
@@ -102,20 +100,29 @@ __device__ __forceinline__ void rd_mlp_layer64(const rd_bf16x8 (&w)[4][2], const
     }
 }
 
-__device__ __forceinline__ void rd_mlp_silu_all(const float (&z)[4][4], float (&h)[4][4])
+// h = SiLU(z), s = sigmoid(z)
+__device__ __forceinline__ void rd_mlp_silu_all(const float (&z)[4][4], float (&s)[4][4], float (&h)[4][4])
 {
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h[b][r] = rd_silu(z[b][r]);
+        for (int r = 0; r < 4; ++r) {
+            s[b][r] = rd_sigmoid(z[b][r]);
+            h[b][r] = z[b][r] * s[b][r];
+        }
 }
 
-// sum over the 16 lanes of a lane group (lanes with equal lane>>4)
+// sum over the 16 lanes of a lane group (lanes with equal lane>>4), in every
+// lane; the order of an xor butterfly over 1, 2, 4, 8, whose last two steps
+// are mirrors here (after two steps the lanes of a quad hold the same sum)
 __device__ __forceinline__ float rd_sum16(float v)
 {
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    v += __shfl_xor(v, 4, 64);
-    v += __shfl_xor(v, 8, 64);
+    auto dpp = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    v += dpp(v, std::integral_constant<int, 0xB1>());      // quad_perm [1,0,3,2]
+    v += dpp(v, std::integral_constant<int, 0x4E>());      // quad_perm [2,3,0,1]
+    v += dpp(v, std::integral_constant<int, 0x141>());     // row_half_mirror
+    v += dpp(v, std::integral_constant<int, 0x140>());     // row_mirror
     return v;
 }

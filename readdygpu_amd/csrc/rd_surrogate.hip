@@ -268,6 +268,17 @@ __device__ __forceinline__ void stage_bf16(__bf16* S, const float (&a)[4][4], in
         for (int r = 0; r < 4; ++r) S[(ti * 16 + 4 * g + r) * RD_TLD + wv * 16 + j] = (__bf16)a[ti][r];
 }
 
+// the same of SiLU = z s
+__device__ __forceinline__ void stage_product(__bf16* S, const float (&z)[4][4], const float (&s)[4][4], int wv, int lane)
+{
+    float h[4][4];
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[ti][r] = z[ti][r] * s[ti][r];
+    stage_bf16(S, h, wv, lane);
+}
+
 __device__ __forceinline__ void stage_f32(float* S, const float (&a)[4][4], int wv, int lane)
 {
     const int j = lane & 15, g = lane >> 4;
@@ -311,7 +322,8 @@ __device__ __forceinline__ void bgrad_rows(const RdTrainStage& S, int ti, float*
 }
 
 // dz of the layer below: (W^T dz) dsilu(z), W^T fragments wt
-__device__ __forceinline__ void back64(const rd_bf16x8 (&wt)[4][2], const float (&z)[4][4], float (&dz)[4][4])
+__device__ __forceinline__ void back64(const rd_bf16x8 (&wt)[4][2], const float (&z)[4][4], const float (&s)[4][4],
+                                       float (&dz)[4][4])
 {
     const rd_f32x4 zero[4] = {};
     float dh[4][4];
@@ -319,7 +331,7 @@ __device__ __forceinline__ void back64(const rd_bf16x8 (&wt)[4][2], const float 
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) dz[b][r] = dh[b][r] * rd_dsilu(z[b][r]);
+        for (int r = 0; r < 4; ++r) dz[b][r] = dh[b][r] * rd_dsilu(z[b][r], s[b][r]);
 }
 
 // Learning rate (cosine from lr0 to lr1 over total steps) and Adam's bias
@@ -339,12 +351,12 @@ struct RdSchedule {
 // registers up front, and the waves meet once per layer, at a stage in LDS
 // (two, used in turn, so that one barrier per stage suffices) from which each
 // wave computes a quarter of the layer's weight and bias gradients.  256
-// steps of 8,192 samples with k_mlp_adam: FIG us a step, against 55 us with
+// steps of 8,192 samples with k_mlp_adam: 16 us a step, against 53 us with
 // 64 samples in each wave (32 workgroups), weights staged in LDS and the step
 // counter in a kernel of its own.  The sums' orders are those of that form.
 // One more workgroup computes the step's schedule meanwhile.
 __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn_all, const float4* __restrict__ tn_all,
-                                                   long m, int batch, int sequential, uint64_t seed,
+                                                   long m, uint64_t inv_m, int batch, int sequential, uint64_t seed,
                                                    const RdMlpPack* __restrict__ pk, RdTrainCtl* __restrict__ ctl,
                                                    float* __restrict__ partial, RdSchedule sch)
 {
@@ -372,7 +384,12 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn
     if (!sequential) {
         uint32_t q[4] = { (uint32_t)c, (uint32_t)step, (uint32_t)(step >> 32), 0x5452414eu };
         philox4x32_10(q, (uint32_t)seed, (uint32_t)(seed >> 32));
-        idx = (long)(((uint64_t)q[1] << 32 | q[0]) % (uint64_t)m);
+        // x mod m from the quotient's estimate mulhi(x, 2^64 / m), at most 2 low
+        const uint64_t x = (uint64_t)q[1] << 32 | q[0];
+        uint64_t rem = x - __umul64hi(x, inv_m) * (uint64_t)m;
+        rem -= rem >= (uint64_t)m ? (uint64_t)m : 0u;
+        rem -= rem >= (uint64_t)m ? (uint64_t)m : 0u;
+        idx = (long)rem;
     }
     if (!live) idx = 0;
     const float4 xa = xn_all[idx], ta = tn_all[idx];
@@ -414,7 +431,7 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn
     const float xn[3] = { xa.x, xa.y, xa.z }, tn[3] = { ta.x, ta.y, ta.z };
 
     // ---- forward ----
-    float z1[4][4], z2[4][4], z3[4][4], h[4][4];
+    float z1[4][4], z2[4][4], z3[4][4], s1[4][4], s2[4][4], s3[4][4], h[4][4];
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
@@ -425,11 +442,11 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn
             v = v + w1[ti][(k + 2) / 4][(k + 2) % 4] * xn[2];
             z1[ti][r] = v + b1[ti][r];
         }
-    rd_mlp_silu_all(z1, h);
+    rd_mlp_silu_all(z1, s1, h);
     rd_mlp_layer64(w2, b2, h, z2);
-    rd_mlp_silu_all(z2, h);
+    rd_mlp_silu_all(z2, s2, h);
     rd_mlp_layer64(w3, b3, h, z3);
-    rd_mlp_silu_all(z3, h);                  // h = h3
+    rd_mlp_silu_all(z3, s3, h);              // h = h3
     rd_f32x4 y = b4;
     y = RD_MFMA(w4[0], rd_mlp_bop(h, 0), y);
     y = RD_MFMA(w4[1], rd_mlp_bop(h, 1), y);
@@ -500,25 +517,23 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float4* __restrict__ xn
             rd_f32x4 acc = { 0.f, 0.f, 0.f, 0.f };
             acc = RD_MFMA(w4t[to], b, acc);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dz[to][r] = acc[r] * rd_dsilu(z3[to][r]);
+            for (int r = 0; r < 4; ++r) dz[to][r] = acc[r] * rd_dsilu(z3[to][r], s3[to][r]);
         }
     }
     // dW3 = dz3 h2^T
-    rd_mlp_silu_all(z2, h);
     stage_bf16(stage[1].d, dz, wv, lane);
-    stage_bf16(stage[1].h, h, wv, lane);
+    stage_product(stage[1].h, z2, s2, wv, lane);
     stage_f32(stage[1].f, dz, wv, lane);
     __syncthreads();
-    back64(w3t, z2, dz);                     // dz2
+    back64(w3t, z2, s2, dz);                   // dz2
     wgrad_rows(stage[1], wv, out + RD_MLP_W3, lane);
     bgrad_rows(stage[1], wv, out + RD_MLP_B3, lane);
     // dW2 = dz2 h1^T
-    rd_mlp_silu_all(z1, h);
     stage_bf16(stage[0].d, dz, wv, lane);
-    stage_bf16(stage[0].h, h, wv, lane);
+    stage_product(stage[0].h, z1, s1, wv, lane);
     stage_f32(stage[0].f, dz, wv, lane);
     __syncthreads();
-    back64(w2t, z1, dz);                     // dz1
+    back64(w2t, z1, s1, dz);                   // dz1
     wgrad_rows(stage[0], wv, out + RD_MLP_W2, lane);
     bgrad_rows(stage[0], wv, out + RD_MLP_B2, lane);
     // dW1 = dz1 xn^T in FP32 on the VALU
@@ -1175,8 +1190,9 @@ static void launch_train_step(rd_system* h, const float4* xn, const float4* tn, 
 {
     const int rows = (batch + 63) / 64;
     const RdSchedule sch = { tp.lr, tp.lr_min, (long long)tp.steps, tp.beta1, tp.beta2 };
-    hipLaunchKernelGGL(k_mlp_train, dim3(rows + 1), dim3(256), 0, h->stream, xn, tn, m, batch, sequential, seed,
-                       (const RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, h->d_partial, sch);
+    hipLaunchKernelGGL(k_mlp_train, dim3(rows + 1), dim3(256), 0, h->stream, xn, tn, m,
+                       ~(uint64_t)0 / (uint64_t)m, batch, sequential, seed, (const RdMlpPack*)h->d_pack,
+                       (RdTrainCtl*)h->d_ctl, h->d_partial, sch);
     hipLaunchKernelGGL(k_mlp_adam, dim3((RD_MLP_NPARAM + 1 + 31) / 32), dim3(256), 0, h->stream, h->d_partial, rows,
                        h->d_master, h->d_mom, h->d_vel, (RdMlpPack*)h->d_pack, (RdTrainCtl*)h->d_ctl, tp.beta1,
                        tp.beta2, tp.eps, grad_out, apply, loss_hist);
