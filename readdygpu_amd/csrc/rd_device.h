@@ -52,6 +52,13 @@ struct RdWave {
     int next;           // first work item of the next replica
 };
 
+// candidate lists of the nearest-piece composite on a regular grid
+struct RdCompGrid {
+    float lo[3], inv[3], edge[3];
+    int n[3];
+    const uint16_t* list;        // null: scan all pieces
+};
+
 // per-system constants, read through one pointer (scalar loads)
 struct RdDev {
     int S;              // pair stencil radius in cells

@@ -145,6 +145,11 @@ struct rd_system {
     bool comp_sum = false;           // RD_COMBINE_SUM: sum of the pieces (else nearest piece)
     int npieces = 0;
     void* d_pieces = nullptr;
+    uint16_t* d_comp_list = nullptr; // candidate lists of the nearest-piece grid (comp_cells cells)
+    long comp_cells = 0;
+    bool comp_grid_set = false;      // built for the pieces and this domain
+    double comp_lo[3] = { 0, 0, 0 }, comp_hi[3] = { 0, 0, 0 };
+    RdCompGrid comp_near{};          // of the step's external pass
     int ext_mode = RD_EXT_EXACT;
     int ext_blocks[2] = { 0, 0 };    // resident workgroups of the exact / surrogate slot passes (0: not yet known)
     float4* d_gext = nullptr;        // external gradient per sorted slot
