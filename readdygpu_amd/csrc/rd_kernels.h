@@ -498,6 +498,7 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
     if (P->n_pot2 > 0) {
         if (P->S == 1 && Lx >= 3 && Ly >= 3 && Lz >= 3) {
             const bool in = interior_cell(R, cx, cy, cz);
+            const bool edge = __any(!in);
             const int lane = threadIdx.x & 63;
             // The walks address the particle array from a copy of its address
             // in vector registers (an identity permutation across the lanes
@@ -549,9 +550,20 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                     dz = min_image(dz, R.Lb[2], R.half[2]);
                 }
             };
+            // the listing needs the magnitudes only: two instructions per axis
+            // (min_image_abs), for every lane of a wave that holds a home at
+            // an edge of the lattice (for the others' candidates in range it
+            // changes nothing: a range is at most a cell, the box at least
+            // three).  Crowded cytosol, 16 replicas: 192 -> 182 us per step
+            // against the branch per lane with the two-sided correction; on
+            // large sparse lattices the same.
             auto test = [&](uint32_t j, float4 q) {           // listing only
-                float dx, dy, dz;
-                delta(q, dx, dy, dz);
+                float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+                if (edge) {
+                    dx = min_image_abs(dx, R.Lb[0]);
+                    dy = min_image_abs(dy, R.Lb[1]);
+                    dz = min_image_abs(dz, R.Lb[2]);
+                }
                 const float d2 = dist2(dx, dy, dz);
                 if (d2 < T.rc2[rowbase + w_type(q.w)] && d2 > 0.0f) {
                     if (nhit < RD_HITS) il->j[nhit][lane] = j;
