@@ -21,12 +21,15 @@
 // Kernels
 // ===========================================================================
 
-// Pack unsorted host input into slot form and histogram the cells.
+// Pack unsorted host input into slot form and histogram the cells.  The
+// tiles' sums are taken from the counts afterwards (k_scan_reduce): a wave of
+// unsorted particles falls in up to 64 tiles, and adding them tile by tile
+// took 185 us at 1M particles (cytosol of 1.26M: 1,030 us), against 50 us (73)
+// for both kernels.
 __global__ __launch_bounds__(RD_BLOCK) void k_pack(const float* __restrict__ xyz, const int* __restrict__ type,
                                                    const int* __restrict__ rep_of, int n,
                                                    const RdRep* __restrict__ reps, float4* __restrict__ pn,
-                                                   uint2* __restrict__ kr,
-                                                   uint32_t* __restrict__ count, uint32_t* __restrict__ tsum,
+                                                   uint2* __restrict__ kr, uint32_t* __restrict__ count,
                                                    uint32_t* __restrict__ gid_n)
 {
     int i = blockIdx.x * RD_BLOCK + threadIdx.x;
@@ -36,7 +39,7 @@ __global__ __launch_bounds__(RD_BLOCK) void k_pack(const float* __restrict__ xyz
     pn[i] = make_float4(x, y, z, w_pack((uint32_t)(i - R.off), type[i]));
     if (gid_n) gid_n[i] = (uint32_t)i;
     uint32_t k = cell_key(R, x, y, z);
-    kr[i] = make_uint2(k, cell_histogram(count, tsum, k));
+    kr[i] = make_uint2(k, atomicAdd(&count[k], 1u));
 }
 
 // wave index and lane of this thread; blocks of RD_BLOCK = 4 waves
@@ -1331,6 +1334,14 @@ static void launch_sort(rd_system* h, int advance)
                        (const uint32_t*)h->d_gid, h->d_slot, h->d_bsum, h->nscan);
 }
 
+// particles of the io arrays into slot form, cell histogram and tile sums
+static void launch_pack(rd_system* h)
+{
+    hipLaunchKernelGGL(k_pack, dim3(nblk(h->n, RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream, h->d_xyz_io, h->d_type_io,
+                       h->d_rep_of, h->n, h->d_reps, h->d_pn, h->d_kr, h->d_count, h->d_gid);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(h->nscan), dim3(RD_BLOCK), 0, h->stream, h->d_count, h->ncell, h->d_bsum);
+}
+
 static int wave_blocks(const rd_system* h) { return std::max(1, nblk(h->nwaves, RD_BLOCK / 64)); }
 
 // ev0/ev1 (measurement only): events the dispatch itself timestamps at the
@@ -1562,8 +1573,7 @@ static int upload(rd_system* h)
             HIPCK(h, hipMemcpyAsync(h->d_type_io, h->htype.data(), sizeof(int) * h->n, hipMemcpyHostToDevice,
                                     h->stream));
         }
-        hipLaunchKernelGGL(k_pack, dim3(nblk(h->n, RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream, h->d_xyz_io, h->d_type_io,
-                           h->d_rep_of, h->n, h->d_reps, h->d_pn, h->d_kr, h->d_count, h->d_bsum, h->d_gid);
+        launch_pack(h);
     }
     launch_sort(h, 0);
     HIPCK(h, hipGetLastError());
@@ -2354,9 +2364,7 @@ extern "C" int rd_frame_rewind(rd_system* h)
     // same particle set and tables: pack the snapshot and sort it again (the
     // captured step graphs stay valid)
     if (h->n > 0)
-        hipLaunchKernelGGL(k_pack, dim3(nblk(h->n, RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream, h->d_xyz_io,
-                           h->d_type_io, h->d_rep_of, h->n, h->d_reps, h->d_pn, h->d_kr, h->d_count,
-                           h->d_bsum, h->d_gid);
+        launch_pack(h);
     launch_sort(h, 0);
     HIPCK(h, hipGetLastError());
     HIPCK(h, hipStreamSynchronize(h->stream));
