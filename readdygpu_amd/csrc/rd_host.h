@@ -123,6 +123,7 @@ struct rd_system {
     size_t pairs_cap = 0;
     uint32_t* d_poff = nullptr;   // per-particle pair offsets and their scan tile sums
     uint32_t* d_pbs = nullptr;
+    uint32_t* d_pkeep = nullptr;  // first partners of each particle
     size_t poff_cap = 0;
 
     // captured steps: one graph per step count
