@@ -69,7 +69,6 @@ struct rd_system {
     float* d_noise = nullptr;
     float* d_xyz_io = nullptr;
     int* d_type_io = nullptr;
-    double* d_etot = nullptr;
     RdRep* d_reps = nullptr;
     RdWave* d_waves = nullptr;
     int* d_rep_of = nullptr;
@@ -126,12 +125,28 @@ struct rd_system {
     uint32_t* d_pkeep = nullptr;  // first partners of each particle
     size_t poff_cap = 0;
 
-    // captured steps: one graph per step count
+    // captured steps: one graph per step count, captured when a count is asked
+    // for the second time
     struct Graph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
+        int asked = 0;
     };
     std::map<int, Graph> graphs;
+
+    // pinned host memory that results pass through (up to RD_STAGE_MAX bytes;
+    // taken from a pool and given back to it)
+    char* hp_stage = nullptr;
+    size_t stage_cap = 0;
+    // reaction lists on the device
+    char* d_react = nullptr;
+    size_t react_cap = 0;
+    // tables as last uploaded
+    RdDev P_up{};
+    bool P_up_set = false;
+    std::vector<RdRep> reps_up;
+    std::vector<RdWave> waves_up;
+    std::vector<RdPot1Dev> pot1_up;
 
     // force-kernel launch configuration (autotuned)
     rd_launch_config lc{};        // requested
@@ -173,6 +188,8 @@ struct rd_system {
     bool ext_active() const { return npieces > 0 || (ext_mode == RD_EXT_SURROGATE && sur_ready); }
 };
 
+#define RD_STAGE_MAX ((size_t)4 << 20)
+char* rd_host_stage(rd_system* h, size_t bytes);
 double rd_host_r0(const rd_system* h, int i, int j);
 int rd_host_refresh(rd_system* h);
 int rd_host_set_step(rd_system* h, uint64_t step);

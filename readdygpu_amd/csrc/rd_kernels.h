@@ -27,6 +27,7 @@ struct RdStepState {
                                     // bit 2: position still outside the box after the periodic
                                     // correction (moved more than one box length in a step),
                                     // bit 3: a pair or bond gradient term beyond the fixed-point range
+    double etot;                    // energy of the last rd_gradients
 };
 
 #define RD_ERR_NONFINITE 1u

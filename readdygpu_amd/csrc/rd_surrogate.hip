@@ -227,15 +227,20 @@ __global__ __launch_bounds__(256) void k_composite_near(const float4* __restrict
     gext[s] = composite_near(g, pieces, np, p.x, p.y, p.z);
 }
 
-// at given points (float4 input, .w ignored)
-__global__ __launch_bounds__(256) void k_composite_points_near(const float4* __restrict__ x, long m, RdCompGrid g,
+__device__ __forceinline__ void put_point(float* __restrict__ grad, float* __restrict__ energy, long i, float4 g)
+{
+    grad[3 * i] = g.x; grad[3 * i + 1] = g.y; grad[3 * i + 2] = g.z;
+    energy[i] = g.w;
+}
+
+// at given points x[3 m]
+__global__ __launch_bounds__(256) void k_composite_points_near(const float* __restrict__ x, long m, RdCompGrid g,
                                                                const RdPiece* __restrict__ pieces, int np,
-                                                               float4* __restrict__ out)
+                                                               float* __restrict__ grad, float* __restrict__ energy)
 {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= m) return;
-    const float4 p = x[i];
-    out[i] = composite_near(g, pieces, np, p.x, p.y, p.z);
+    put_point(grad, energy, i, composite_near(g, pieces, np, x[3 * i], x[3 * i + 1], x[3 * i + 2]));
 }
 
 // exact pass over sorted slots: gext[s] for the particles whose type is in the
@@ -302,19 +307,18 @@ __global__ __launch_bounds__(256) void k_composite_all(const float4* __restrict_
     gext[s] = composite_at<SUM>(pc, np, p.x, p.y, p.z);
 }
 
-// exact evaluation at given points (float4 input, .w ignored)
+// exact evaluation at given points x[3 m]
 template <bool SUM>
-__global__ __launch_bounds__(256) void k_composite_points(const float4* __restrict__ x, long m,
+__global__ __launch_bounds__(256) void k_composite_points(const float* __restrict__ x, long m,
                                                           const RdPiece* __restrict__ pieces, int np,
-                                                          float4* __restrict__ out)
+                                                          float* __restrict__ grad, float* __restrict__ energy)
 {
     extern __shared__ RdPiece pc[];
     for (int k = threadIdx.x; k < np; k += 256) pc[k] = pieces[k];
     __syncthreads();
-    long i = (long)blockIdx.x * 256 + threadIdx.x;
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= m) return;
-    float4 p = x[i];
-    out[i] = composite_at<SUM>(pc, np, p.x, p.y, p.z);
+    put_point(grad, energy, i, composite_at<SUM>(pc, np, x[3 * i], x[3 * i + 1], x[3 * i + 2]));
 }
 
 // ===========================================================================
@@ -984,9 +988,11 @@ __global__ __launch_bounds__(256) void k_mlp_slots(const RdMlpPack* __restrict__
     if (tail != head) tile(head, (int)(tail - head));
 }
 
-// inference at normalised points (float4 xn) -> raw network output (float4)
-__global__ __launch_bounds__(256) void k_mlp_points(const RdMlpPack* __restrict__ pk, const float4* __restrict__ xin,
-                                                    long m, float4* __restrict__ out)
+// inference at normalised points -> raw network output, STRIDE values per
+// point in both (3, or 4 with the last one unused)
+template <int STRIDE>
+__global__ __launch_bounds__(256) void k_mlp_points(const RdMlpPack* __restrict__ pk, const float* __restrict__ xin,
+                                                    long m, float* __restrict__ out)
 {
     __shared__ RdMlpFwdLds L;
     mlp_stage<256>(L, pk);
@@ -997,10 +1003,40 @@ __global__ __launch_bounds__(256) void k_mlp_points(const RdMlpPack* __restrict_
     const long stride = (long)gridDim.x * wpb;
     for (long t = (long)xcd_block(blockIdx.x, gridDim.x) * wpb + (threadIdx.x >> 6); t < ntiles; t += stride) {
         const long i = t * 16 + j;
-        const float4 p = i < m ? xin[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        float xn[3] = { p.x, p.y, p.z };
+        float xn[3] = { 0.f, 0.f, 0.f };
+        if (i < m) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) xn[k] = xin[i * STRIDE + k];
+        }
         const float3 y = mlp_tile(L, xn);
-        if (lane < 16 && i < m) out[i] = make_float4(y.x, y.y, y.z, 0.f);
+        if (lane < 16 && i < m) {
+            out[i * STRIDE] = y.x; out[i * STRIDE + 1] = y.y; out[i * STRIDE + 2] = y.z;
+        }
+    }
+}
+
+// squared error of the network's outputs y (times gscale) against the exact
+// gradients t, and the squared gradients, per workgroup in FP64
+__global__ __launch_bounds__(256) void k_sur_error(const float4* __restrict__ t, const float4* __restrict__ y, long m,
+                                                   double gscale, double* __restrict__ num, double* __restrict__ den)
+{
+    __shared__ double red[2][4];
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    double a = 0.0, b = 0.0;
+    if (i < m) {
+        const float4 g = t[i], v = y[i];
+        const double ex = g.x, ey = g.y, ez = g.z;
+        const double dx = v.x * gscale - ex, dy = v.y * gscale - ey, dz = v.z * gscale - ez;
+        a = dx * dx + dy * dy + dz * dz;
+        b = ex * ex + ey * ey + ez * ez;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { a += __shfl_down(a, o, 64); b += __shfl_down(b, o, 64); }
+    if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x >> 6] = a; red[1][threadIdx.x >> 6] = b; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        num[blockIdx.x] = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+        den[blockIdx.x] = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     }
 }
 
@@ -1220,6 +1256,32 @@ extern "C" int rd_set_external_mode(rd_system* h, int mode)
     return RD_OK;
 }
 
+// Points to the device, and results (a[na], then b[nb] in one device array; a
+// null destination is left out) back, through pinned memory where it holds
+// them; points_out waits for the stream.
+static hipError_t points_in(rd_system* h, float* dst, const float* src, long n)
+{
+    char* stage = rd_host_stage(h, sizeof(float) * (size_t)n);
+    if (stage) memcpy(stage, src, sizeof(float) * (size_t)n);
+    return hipMemcpyAsync(dst, stage ? (const void*)stage : (const void*)src, sizeof(float) * (size_t)n,
+                          hipMemcpyHostToDevice, h->stream);
+}
+
+static hipError_t points_out(rd_system* h, float* a, long na, float* b, long nb, const float* src)
+{
+    // (the pinned memory may still feed the copy of the points)
+    hipError_t e = hipStreamSynchronize(h->stream);
+    const size_t sa = sizeof(float) * (size_t)na, sb = sizeof(float) * (size_t)nb;
+    char* stage = e == hipSuccess ? rd_host_stage(h, sa + sb) : nullptr;
+    if (e == hipSuccess && stage) e = hipMemcpyAsync(stage, src, sa + sb, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess && !stage && a) e = hipMemcpyAsync(a, src, sa, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess && !stage && b) e = hipMemcpyAsync(b, src + na, sb, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess && stage && a) memcpy(a, stage, sa);
+    if (e == hipSuccess && stage && b) memcpy(b, stage + sa, sb);
+    return e;
+}
+
 // exact composite at host points (test and data checks)
 extern "C" int rd_composite_eval(rd_system* h, long m, const float* xyz, float* grad, float* energy)
 {
@@ -1229,31 +1291,24 @@ extern "C" int rd_composite_eval(rd_system* h, long m, const float* xyz, float* 
     RdCompGrid g;
     const int rc = comp_grid(h, &g);
     if (rc) return rc;
-    std::vector<float4> x(m), o(m);
-    for (long i = 0; i < m; ++i) x[i] = make_float4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0.f);
-    float4 *dx = nullptr, *dout = nullptr;
-    SHIPCK(h, hipMalloc(&dx, sizeof(float4) * m));
-    hipError_t e = hipMalloc(&dout, sizeof(float4) * m);
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, x.data(), sizeof(float4) * m, hipMemcpyHostToDevice, h->stream);
+    float *dx = nullptr, *dg = nullptr;                 // positions; gradients, then energies
+    SHIPCK(h, hipMalloc(&dx, sizeof(float) * 3 * m));
+    hipError_t e = hipMalloc(&dg, sizeof(float) * 4 * m);
+    if (e == hipSuccess) e = points_in(h, dx, xyz, 3 * m);
     if (e == hipSuccess) {
         if (g.list)
             hipLaunchKernelGGL(k_composite_points_near, dim3(nb256(m)), dim3(256), 0, h->stream, dx, m, g,
-                               (const RdPiece*)h->d_pieces, h->npieces, dout);
+                               (const RdPiece*)h->d_pieces, h->npieces, dg, dg + 3 * m);
         else
             hipLaunchKernelGGL(h->comp_sum ? k_composite_points<true> : k_composite_points<false>, dim3(nb256(m)),
                                dim3(256), pieces_lds(h), h->stream, dx, m, (const RdPiece*)h->d_pieces, h->npieces,
-                               dout);
+                               dg, dg + 3 * m);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(o.data(), dout, sizeof(float4) * m, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = points_out(h, grad, 3 * m, energy, m, dg);
     (void)hipFree(dx);
-    if (dout) (void)hipFree(dout);
+    if (dg) (void)hipFree(dg);
     if (e != hipSuccess) return sset_err(h, RD_EHIP, std::string("composite eval: ") + hipGetErrorString(e));
-    for (long i = 0; i < m; ++i) {
-        if (grad) { grad[3 * i] = o[i].x; grad[3 * i + 1] = o[i].y; grad[3 * i + 2] = o[i].z; }
-        if (energy) energy[i] = o[i].w;
-    }
     return RD_OK;
 }
 
@@ -1495,29 +1550,16 @@ extern "C" int rd_surrogate_train(rd_system* h, const rd_train_params* tp, float
     SHIPCK(h, hipMemset(h->d_ctl, 0, sizeof(RdTrainCtl)));
     SHIPCK(h, hipMemset(h->d_mom, 0, sizeof(float) * RD_MLP_NPARAM));
     SHIPCK(h, hipMemset(h->d_vel, 0, sizeof(float) * RD_MLP_NPARAM));
-    // capture a block of steps once and replay it
-    const int chunk = tp->steps >= 64 ? 64 : tp->steps;
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    SHIPCK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < chunk; ++i)
-        launch_train_step(h, h->d_xn, h->d_tg, h->nsamples, tp->batch, 0, tp->seed, *tp, nullptr, 1, h->d_loss_hist);
-    SHIPCK(h, hipStreamEndCapture(h->stream, &g));
-    hipError_t e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    int done = 0;
-    while (e == hipSuccess && done + chunk <= tp->steps) {
-        e = hipGraphLaunch(ge, h->stream);
-        done += chunk;
-    }
-    for (; e == hipSuccess && done < tp->steps; ++done) {
+    // two launches a step, 5 us of host time against 16 us on the GPU (a graph
+    // of 64 steps took 0.7 ms to capture, instantiate and free)
+    hipError_t e = hipSuccess;
+    for (int done = 0; e == hipSuccess && done < tp->steps; ++done) {
         launch_train_step(h, h->d_xn, h->d_tg, h->nsamples, tp->batch, 0, tp->seed, *tp, nullptr, 1, h->d_loss_hist);
         e = hipGetLastError();
     }
     if (e == hipSuccess && loss_curve)
         e = hipMemcpyAsync(loss_curve, h->d_loss_hist, sizeof(float) * tp->steps, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (ge) (void)hipGraphExecDestroy(ge);
-    if (g) (void)hipGraphDestroy(g);
     if (e != hipSuccess) return sset_err(h, RD_EHIP, std::string("train: ") + hipGetErrorString(e));
     h->dirty = true;     // new packed weights: the captured step graphs stay valid (same buffers)
     return RD_OK;
@@ -1529,23 +1571,19 @@ extern "C" int rd_surrogate_predict(rd_system* h, long m, const float* xn, float
     if (!h || m < 0 || (m > 0 && (!xn || !y))) return RD_EINVAL;
     if (!h->sur_ready) return sset_err(h, RD_ESTATE, "the surrogate has no weights");
     if (m == 0) return RD_OK;
-    std::vector<float4> hx(m), ho(m);
-    for (long i = 0; i < m; ++i) hx[i] = make_float4(xn[3 * i], xn[3 * i + 1], xn[3 * i + 2], 0.f);
-    float4 *dx = nullptr, *dout = nullptr;
-    SHIPCK(h, hipMalloc(&dx, sizeof(float4) * m));
-    hipError_t e = hipMalloc(&dout, sizeof(float4) * m);
-    if (e == hipSuccess) e = hipMemcpyAsync(dx, hx.data(), sizeof(float4) * m, hipMemcpyHostToDevice, h->stream);
+    float *dx = nullptr, *dout = nullptr;
+    SHIPCK(h, hipMalloc(&dx, sizeof(float) * 3 * m));
+    hipError_t e = hipMalloc(&dout, sizeof(float) * 3 * m);
+    if (e == hipSuccess) e = points_in(h, dx, xn, 3 * m);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_mlp_points, dim3(mlp_point_blocks(m)), dim3(256), 0, h->stream,
-                           (const RdMlpPack*)h->d_pack, (const float4*)dx, m, dout);
+        hipLaunchKernelGGL(k_mlp_points<3>, dim3(mlp_point_blocks(m)), dim3(256), 0, h->stream,
+                           (const RdMlpPack*)h->d_pack, (const float*)dx, m, dout);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(ho.data(), dout, sizeof(float4) * m, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = points_out(h, y, 3 * m, nullptr, 0, dout);
     (void)hipFree(dx);
     if (dout) (void)hipFree(dout);
     if (e != hipSuccess) return sset_err(h, RD_EHIP, std::string("predict: ") + hipGetErrorString(e));
-    for (long i = 0; i < m; ++i) { y[3 * i] = ho[i].x; y[3 * i + 1] = ho[i].y; y[3 * i + 2] = ho[i].z; }
     return RD_OK;
 }
 
@@ -1555,36 +1593,34 @@ extern "C" int rd_surrogate_validate(rd_system* h, long m, uint64_t seed, double
 {
     if (!h || m < 64 || !rel_rmse) return RD_EINVAL;
     if (!h->sur_ready || h->npieces <= 0) return sset_err(h, RD_ESTATE, "composite and surrogate required");
-    float4 *dx = nullptr, *dt = nullptr, *dy = nullptr;
-    double* bs = nullptr;
-    float* gs = nullptr;
-    SHIPCK(h, hipMalloc(&dx, sizeof(float4) * m));
-    SHIPCK(h, hipMalloc(&dt, sizeof(float4) * m));
-    SHIPCK(h, hipMalloc(&dy, sizeof(float4) * m));
-    SHIPCK(h, hipMalloc(&bs, sizeof(double) * nb256(m)));
-    const RdMlpNorm& nm = h->mlp_norm;
-    if (launch_sur_data(h, m, seed, dx, dt, bs) != RD_OK) {
-        (void)hipFree(dx); (void)hipFree(dt); (void)hipFree(dy); (void)hipFree(bs);
-        return RD_EHIP;
+    const unsigned nb = nb256(m);
+    float4* d = nullptr;                             // positions, exact gradients, outputs
+    double* bs = nullptr;                            // sums of each workgroup (two sets)
+    SHIPCK(h, hipMalloc(&d, sizeof(float4) * 3 * m));
+    hipError_t e = hipMalloc(&bs, sizeof(double) * 2 * nb);
+    int rc = RD_OK;
+    std::vector<double> sums(2 * (size_t)nb);
+    if (e == hipSuccess) {
+        float4 *dt = d + m, *dy = d + 2 * m;
+        rc = launch_sur_data(h, m, seed, d, dt, bs);
+        if (rc == RD_OK) {
+            hipLaunchKernelGGL(k_mlp_points<4>, dim3(mlp_point_blocks(m)), dim3(256), 0, h->stream,
+                               (const RdMlpPack*)h->d_pack, (const float*)d, m, (float*)dy);
+            hipLaunchKernelGGL(k_sur_error, dim3(nb), dim3(256), 0, h->stream, dt, dy, m, (double)h->mlp_norm.gscale,
+                               bs, bs + nb);
+            e = hipGetLastError();
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(sums.data(), bs, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost, h->stream);
+        }
+        const hipError_t se = hipStreamSynchronize(h->stream);
+        if (e == hipSuccess) e = se;
     }
-    hipLaunchKernelGGL(k_mlp_points, dim3(mlp_point_blocks(m)), dim3(256), 0, h->stream, (const RdMlpPack*)h->d_pack,
-                       (const float4*)dx, m, dy);
-    hipError_t e = hipGetLastError();
-    std::vector<float4> t(m), y(m);
-    if (e == hipSuccess) e = hipMemcpyAsync(t.data(), dt, sizeof(float4) * m, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(y.data(), dy, sizeof(float4) * m, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(dx); (void)hipFree(dt); (void)hipFree(dy); (void)hipFree(bs);
-    (void)gs;
+    (void)hipFree(d);
+    if (bs) (void)hipFree(bs);
+    if (rc) return rc;
     if (e != hipSuccess) return sset_err(h, RD_EHIP, std::string("validate: ") + hipGetErrorString(e));
     double num = 0.0, den = 0.0;
-    const double sc = nm.gscale;
-    for (long i = 0; i < m; ++i) {
-        double ex = t[i].x, ey = t[i].y, ez = t[i].z;
-        double dxv = y[i].x * sc - ex, dyv = y[i].y * sc - ey, dzv = y[i].z * sc - ez;
-        num += dxv * dxv + dyv * dyv + dzv * dzv;
-        den += ex * ex + ey * ey + ez * ez;
-    }
+    for (unsigned i = 0; i < nb; ++i) { num += sums[i]; den += sums[nb + i]; }
     *rel_rmse = den > 0 ? std::sqrt(num / den) : 0.0;
     return RD_OK;
 }

@@ -762,7 +762,8 @@ __global__ __launch_bounds__(RD_BLOCK) void k_rdf_global(const float4* __restric
 // index and keeps the first RD_PAIR_KEEP partners of each particle; an
 // exclusive scan turns the counts into offsets; k_pairs_emit writes each
 // particle's pairs into its own segment, sorted by j, from the kept partners,
-// or walks the stencil again for a particle with more.
+// or walks the stencil again for a particle with more.  Segments past `cap`
+// pairs are left out (the caller grows the list and emits again).
 // 1M particles, 241,000 pairs: find 35 + emit 16 us against 50 + 52 for two full walks
 // (count, then emit).
 #define RD_PAIR_KEEP 4
@@ -831,7 +832,7 @@ __global__ __launch_bounds__(RD_BLOCK) void k_pairs_emit(const float4* __restric
                                                          const RdWave* __restrict__ waves, int nwaves,
                                                          const float* __restrict__ thr2, int S,
                                                          const uint32_t* __restrict__ off,
-                                                         const uint32_t* __restrict__ keep, PairT* __restrict__ out)
+                                                         const uint32_t* __restrict__ keep, PairT* __restrict__ out, uint32_t cap)
 {
     const RdWave it = wave_item(waves, nwaves, wave_id());
     const int s = it.s0 + (threadIdx.x & 63);
@@ -840,7 +841,7 @@ __global__ __launch_bounds__(RD_BLOCK) void k_pairs_emit(const float4* __restric
     // that the offsets are read in order)
     if (keep) {
         const uint32_t gi = (uint32_t)s, o = off[gi], n = off[gi + 1] - o;
-        if (n > 0 && n <= RD_PAIR_KEEP) {
+        if (n > 0 && n <= RD_PAIR_KEEP && o + n <= cap) {
             static_assert(RD_PAIR_KEEP == 4, "four kept partners are sorted");
             const uint4 v = *reinterpret_cast<const uint4*>(keep + (size_t)gi * RD_PAIR_KEEP);
             uint32_t a = v.x, b = n > 1 ? v.y : ~0u, c = n > 2 ? v.z : ~0u, d = n > 3 ? v.w : ~0u;
@@ -855,7 +856,7 @@ __global__ __launch_bounds__(RD_BLOCK) void k_pairs_emit(const float4* __restric
     const float4 p = ps[s];
     const RdRep R = reps[it.rep];
     const uint32_t ii = w_index(p.w), gi = (uint32_t)R.off + ii, o = off[gi], n = off[gi + 1] - o;
-    if (n <= (keep ? (uint32_t)RD_PAIR_KEEP : 0u)) return;
+    if (n <= (keep ? (uint32_t)RD_PAIR_KEEP : 0u) || o + n > cap) return;
     const int nt = P->nt, ti = w_type(p.w);
     int cx, cy, cz;
     cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
@@ -908,6 +909,78 @@ static int step_error(rd_system* h, unsigned int err)
 
 static inline int nblk(long n, int b) { return (int)((n + b - 1) / b); }
 
+// Pinned host memory for results.  A copy from the device into it is one
+// transfer: 24 KB take 8 us with the wait against 18 us into pageable memory,
+// 160 KB 11 against 75, 4 MB 82 against 239, before the copy to the caller.
+// But the host's first touch of new pinned pages costs 1.5 us a page (2 MB:
+// 0.8 ms), so buffers go from handle to handle through a pool of at most
+// RD_POOL_MAX bytes, and larger results (16 MB: 843 us against 955) take the
+// pageable way, straight into the caller's memory.
+#define RD_POOL_MAX ((size_t)16 << 20)
+struct RdPinned {
+    char* p;
+    size_t cap;
+};
+static std::mutex pool_mu;
+static std::vector<RdPinned> pool_free;
+
+static void stage_release(rd_system* h)
+{
+    if (!h->hp_stage) return;
+    const RdPinned b = { h->hp_stage, h->stage_cap };
+    h->hp_stage = nullptr;
+    h->stage_cap = 0;
+    {
+        std::lock_guard<std::mutex> lock(pool_mu);
+        size_t held = 0;
+        for (const RdPinned& q : pool_free) held += q.cap;
+        if (held + b.cap <= RD_POOL_MAX) {
+            pool_free.push_back(b);
+            return;
+        }
+    }
+    (void)hipHostFree(b.p);
+}
+
+// At least `bytes` of it (null beyond RD_STAGE_MAX or when there is none).
+// Every entry point that uses it waits for the stream before it returns.
+char* rd_host_stage(rd_system* h, size_t bytes)
+{
+    if (bytes > RD_STAGE_MAX) return nullptr;
+    if (bytes <= h->stage_cap) return h->hp_stage;
+    stage_release(h);
+    {
+        std::lock_guard<std::mutex> lock(pool_mu);
+        int best = -1;
+        for (int i = 0; i < (int)pool_free.size(); ++i)
+            if (pool_free[i].cap >= bytes && (best < 0 || pool_free[i].cap < pool_free[best].cap)) best = i;
+        if (best >= 0) {
+            h->hp_stage = pool_free[best].p;
+            h->stage_cap = pool_free[best].cap;
+            pool_free.erase(pool_free.begin() + best);
+            return h->hp_stage;
+        }
+    }
+    const size_t cap = std::min(std::max(bytes + bytes / 4, (size_t)64 << 10), RD_STAGE_MAX);
+    if (hipHostMalloc((void**)&h->hp_stage, cap, hipHostMallocDefault) != hipSuccess) {
+        h->hp_stage = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    h->stage_cap = cap;
+    return h->hp_stage;
+}
+
+// the device's step state, after everything enqueued so far
+static int read_state(rd_system* h, RdStepState* st)
+{
+    char* p = rd_host_stage(h, sizeof(*st));
+    HIPCK(h, hipMemcpyAsync(p ? (void*)p : (void*)st, h->d_st, sizeof(*st), hipMemcpyDeviceToHost, h->stream));
+    HIPCK(h, hipStreamSynchronize(h->stream));
+    if (p) memcpy(st, p, sizeof(*st));
+    return RD_OK;
+}
+
 static void drop_graph(rd_system* h)
 {
     for (auto& kv : h->graphs) {
@@ -948,7 +1021,7 @@ static void free_dev(rd_system* h)
     void* ptrs[] = { h->d_ps, h->d_pn, h->d_kr, h->d_count, h->d_start, h->d_bsum,
                      h->d_P, h->d_pot1, h->d_st, h->d_noise, h->d_rdf, h->d_rdf_part, h->d_pairs,
                      h->d_poff, h->d_pbs, h->d_pkeep,
-                     h->d_xyz_io, h->d_type_io, h->d_etot, h->d_reps, h->d_waves, h->d_rep_of };
+                     h->d_xyz_io, h->d_type_io, h->d_reps, h->d_waves, h->d_rep_of, h->d_react };
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     h->d_ps = h->d_pn = nullptr;
@@ -957,7 +1030,9 @@ static void free_dev(rd_system* h)
     h->d_P = nullptr; h->d_pot1 = nullptr; h->d_st = nullptr; h->d_noise = nullptr;
     h->d_rdf = nullptr; h->d_rdf_part = nullptr; h->d_pairs = nullptr;
     h->d_poff = nullptr; h->d_pbs = nullptr; h->d_pkeep = nullptr; h->poff_cap = 0;
-    h->d_xyz_io = nullptr; h->d_type_io = nullptr; h->d_etot = nullptr;
+    h->d_xyz_io = nullptr; h->d_type_io = nullptr; h->d_react = nullptr; h->react_cap = 0;
+    stage_release(h);
+    h->P_up_set = false; h->reps_up.clear(); h->waves_up.clear(); h->pot1_up.clear();
     h->d_reps = nullptr; h->d_waves = nullptr; h->d_rep_of = nullptr;
     h->cap = 0; h->ncell_alloc = 0; h->pairs_cap = 0; h->noise_cap = 0; h->nrep_alloc = 0; h->nwave_alloc = 0;
 }
@@ -1322,10 +1397,11 @@ static int grow_particles(rd_system* h, int need, bool keep_ps)
             if (p) (void)hipFree(p);
         h->d_pn = nullptr; h->d_kr = nullptr; h->d_xyz_io = nullptr; h->d_type_io = nullptr;
         h->d_rep_of = nullptr;
+        h->waves_up.clear();             // (k_rep_of runs again)
         h->d_ps = nps;
         HIPCK(h, hipMalloc(&h->d_pn, sizeof(float4) * cap));
         HIPCK(h, hipMalloc(&h->d_kr, sizeof(uint2) * cap));
-        HIPCK(h, hipMalloc(&h->d_xyz_io, sizeof(float) * 3 * cap));
+        HIPCK(h, hipMalloc(&h->d_xyz_io, sizeof(float) * 4 * cap));    // positions, then types of a copy to the host
         HIPCK(h, hipMalloc(&h->d_type_io, sizeof(int) * cap));
         HIPCK(h, hipMalloc(&h->d_rep_of, sizeof(int) * cap));
         h->cap = cap;
@@ -1357,16 +1433,21 @@ static int ensure_capacity(rd_system* h)
     if ((int)h->rep_dev.size() > h->nrep_alloc) {
         drop_graph(h);
         if (h->d_reps) (void)hipFree(h->d_reps);
+        h->reps_up.clear();
         HIPCK(h, hipMalloc(&h->d_reps, sizeof(RdRep) * h->rep_dev.size()));
         h->nrep_alloc = (int)h->rep_dev.size();
     }
     if (std::max(h->nwaves, 1) > h->nwave_alloc) {
         drop_graph(h);
         if (h->d_waves) (void)hipFree(h->d_waves);
+        h->waves_up.clear();
         HIPCK(h, hipMalloc(&h->d_waves, sizeof(RdWave) * std::max(h->nwaves, 1)));
         h->nwave_alloc = std::max(h->nwaves, 1);
     }
-    if (!h->d_P) HIPCK(h, hipMalloc(&h->d_P, sizeof(RdDev)));
+    if (!h->d_P) {
+        HIPCK(h, hipMalloc(&h->d_P, sizeof(RdDev)));
+        h->P_up_set = false;
+    }
     if (!h->d_st) {
         HIPCK(h, hipMalloc(&h->d_st, sizeof(RdStepState)));
         RdStepState s0;
@@ -1374,7 +1455,6 @@ static int ensure_capacity(rd_system* h)
         s0.step = h->step;
         HIPCK(h, hipMemcpyAsync(h->d_st, &s0, sizeof(s0), hipMemcpyHostToDevice, h->stream));
     }
-    if (!h->d_etot) HIPCK(h, hipMalloc(&h->d_etot, sizeof(double)));
     return RD_OK;
 }
 
@@ -1599,12 +1679,28 @@ static int upload(rd_system* h)
     h->kern = h->lc.kernel == RD_KERNEL_QUEUE ? RD_KERNEL_QUEUE : RD_KERNEL_GATHER;
     h->block = (h->lc.block == 64 || h->lc.block == 128 || h->lc.block == 512) ? h->lc.block : 256;
     h->ppt = (h->lc.ppt == 2 || h->lc.ppt == 4) ? h->lc.ppt : 1;
-    HIPCK(h, hipMemcpyAsync(h->d_P, &h->P, sizeof(RdDev), hipMemcpyHostToDevice, h->stream));
-    HIPCK(h, hipMemcpyAsync(h->d_reps, h->rep_dev.data(), sizeof(RdRep) * h->rep_dev.size(), hipMemcpyHostToDevice,
-                            h->stream));
-    if (h->nwaves > 0)
-        HIPCK(h, hipMemcpyAsync(h->d_waves, h->wave_tab.data(), sizeof(RdWave) * h->nwaves, hipMemcpyHostToDevice,
+    // tables whose bytes are those of the last upload stay (a copy from
+    // pageable memory costs 10 us or more)
+    auto same = [](const auto& a, const auto& b) {
+        return a.size() == b.size() && (a.empty() || memcmp(a.data(), b.data(), sizeof(a[0]) * a.size()) == 0);
+    };
+    if (!h->P_up_set || memcmp(&h->P, &h->P_up, sizeof(RdDev)) != 0) {
+        memcpy(&h->P_up, &h->P, sizeof(RdDev));
+        HIPCK(h, hipMemcpyAsync(h->d_P, &h->P_up, sizeof(RdDev), hipMemcpyHostToDevice, h->stream));
+        h->P_up_set = true;
+    }
+    if (!same(h->reps_up, h->rep_dev)) {
+        h->reps_up = h->rep_dev;
+        HIPCK(h, hipMemcpyAsync(h->d_reps, h->reps_up.data(), sizeof(RdRep) * h->reps_up.size(), hipMemcpyHostToDevice,
                                 h->stream));
+    }
+    const bool new_waves = !same(h->waves_up, h->wave_tab);
+    if (new_waves) {
+        h->waves_up = h->wave_tab;
+        if (h->nwaves > 0)
+            HIPCK(h, hipMemcpyAsync(h->d_waves, h->waves_up.data(), sizeof(RdWave) * h->nwaves, hipMemcpyHostToDevice,
+                                    h->stream));
+    }
     if (h->noise_n >= 0 && h->noise_n != h->n) {
         // the noise array was laid out for another particle count: back to the generator
         RdStepState st;
@@ -1614,16 +1710,20 @@ static int upload(rd_system* h)
         HIPCK(h, hipMemcpyAsync(h->d_st, &st, sizeof(st), hipMemcpyHostToDevice, h->stream));
         h->noise_n = -1;
     }
-    if (h->d_pot1) { (void)hipFree(h->d_pot1); h->d_pot1 = nullptr; }
-    if (!h->pot1dev.empty()) {
-        HIPCK(h, hipMalloc(&h->d_pot1, sizeof(RdPot1Dev) * h->pot1dev.size()));
-        HIPCK(h, hipMemcpyAsync(h->d_pot1, h->pot1dev.data(), sizeof(RdPot1Dev) * h->pot1dev.size(),
-                                hipMemcpyHostToDevice, h->stream));
+    if (!same(h->pot1_up, h->pot1dev)) {
+        if (h->d_pot1) { (void)hipFree(h->d_pot1); h->d_pot1 = nullptr; }
+        h->pot1_up = h->pot1dev;
+        if (!h->pot1_up.empty()) {
+            HIPCK(h, hipMalloc(&h->d_pot1, sizeof(RdPot1Dev) * h->pot1_up.size()));
+            HIPCK(h, hipMemcpyAsync(h->d_pot1, h->pot1_up.data(), sizeof(RdPot1Dev) * h->pot1_up.size(),
+                                    hipMemcpyHostToDevice, h->stream));
+        }
     }
     if (h->n > 0) {
         // replica of each particle index: the wave table covers the same ranges
-        hipLaunchKernelGGL(k_rep_of, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_waves, h->nwaves,
-                           h->d_rep_of);
+        if (new_waves)
+            hipLaunchKernelGGL(k_rep_of, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_waves, h->nwaves,
+                               h->d_rep_of);
         if (!h->io_on_device) {
             HIPCK(h, hipMemcpyAsync(h->d_xyz_io, h->hxyz.data(), sizeof(float) * 3 * h->n, hipMemcpyHostToDevice,
                                     h->stream));
@@ -1672,9 +1772,8 @@ static int refresh(rd_system* h)
 // One hipGraph per step count: K steps captured once, launched as one graph.
 static int step_graph(rd_system* h, int k, hipGraphExec_t* exec)
 {
-    auto it = h->graphs.find(k);
-    if (it != h->graphs.end()) { *exec = it->second.exec; return RD_OK; }
-    rd_system::Graph gr;
+    rd_system::Graph& gr = h->graphs[k];
+    if (gr.exec) { *exec = gr.exec; return RD_OK; }
     HIPCK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     for (int i = 0; i < k; ++i) launch_step(h);
     hipError_t e = hipStreamEndCapture(h->stream, &gr.graph);
@@ -1682,23 +1781,33 @@ static int step_graph(rd_system* h, int k, hipGraphExec_t* exec)
     e = hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(gr.graph);
+        gr.graph = nullptr;
+        gr.exec = nullptr;
         return set_err(h, RD_EHIP, std::string("graph instantiate: ") + hipGetErrorString(e));
     }
-    h->graphs[k] = gr;
     *exec = gr.exec;
     return RD_OK;
 }
 
-// launch nsteps steps as graphs of up to RD_GRAPH_STEPS steps
+// Launch nsteps steps, in graphs of 256 and 16 steps and single launches.  A
+// graph is captured when its step count is asked for the second time since the
+// tables changed: capturing and instantiating 16 steps takes 430 us (256:
+// 2.8 ms), more than launching them (110 us), which a program that changes
+// its particles every frame would pay each time.  A graph of one step takes
+// 20 us longer to start than its three launches.
 static int launch_steps(rd_system* h, int nsteps)
 {
-    const int chunk = 256;
     while (nsteps > 0) {
-        int k = nsteps >= chunk ? chunk : (nsteps >= 16 ? 16 : 1);
-        hipGraphExec_t ex;
-        int rc = step_graph(h, k, &ex);
-        if (rc) return rc;
-        HIPCK(h, hipGraphLaunch(ex, h->stream));
+        const int k = nsteps >= 256 ? 256 : (nsteps >= 16 ? 16 : nsteps);
+        if (k >= 16 && h->graphs[k].asked++ > 0) {
+            hipGraphExec_t ex;
+            int rc = step_graph(h, k, &ex);
+            if (rc) return rc;
+            HIPCK(h, hipGraphLaunch(ex, h->stream));
+        } else {
+            for (int i = 0; i < k; ++i) launch_step(h);
+            HIPCK(h, hipGetLastError());
+        }
         nsteps -= k;
         h->step += (uint64_t)k;
     }
@@ -1714,9 +1823,8 @@ extern "C" int rd_simulate(rd_system* h, int nsteps)
     rc = launch_steps(h, nsteps);
     if (rc) return rc;
     RdStepState st;
-    HIPCK(h, hipMemcpyAsync(&st, h->d_st, sizeof(st), hipMemcpyDeviceToHost, h->stream));
-    HIPCK(h, hipStreamSynchronize(h->stream));
-    return step_error(h, st.err);
+    rc = read_state(h, &st);
+    return rc ? rc : step_error(h, st.err);
 }
 
 // pieces of the step for the measurement entry points (rd_bench.hip)
@@ -1781,15 +1889,28 @@ extern "C" int rd_copy_pos_from_device(rd_system* h, float* xyz, int* type)
         return RD_OK;
     }
     HIPCK(h, hipSetDevice(h->dev));
-    if (h->n > 0) {
+    const size_t n = (size_t)h->n;
+    if (n > 0) {
+        // types behind the positions, so that one copy brings both; without a
+        // destination the host mirrors are refreshed
+        int* dtype = (int*)(h->d_xyz_io + 3 * n);
         hipLaunchKernelGGL(k_unsort, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_reps,
-                           h->d_waves, h->nwaves, h->d_xyz_io, h->d_type_io);
-        HIPCK(h, hipMemcpyAsync(h->hxyz.data(), h->d_xyz_io, sizeof(float) * 3 * h->n, hipMemcpyDeviceToHost, h->stream));
-        HIPCK(h, hipMemcpyAsync(h->htype.data(), h->d_type_io, sizeof(int) * h->n, hipMemcpyDeviceToHost, h->stream));
+                           h->d_waves, h->nwaves, h->d_xyz_io, dtype);
+        HIPCK(h, hipGetLastError());
+        if (!xyz && !type) { xyz = h->hxyz.data(); type = h->htype.data(); }
+        char* stage = rd_host_stage(h, 16 * n);
+        if (stage) {
+            HIPCK(h, hipMemcpyAsync(stage, h->d_xyz_io, 16 * n, hipMemcpyDeviceToHost, h->stream));
+        } else {
+            if (xyz) HIPCK(h, hipMemcpyAsync(xyz, h->d_xyz_io, 12 * n, hipMemcpyDeviceToHost, h->stream));
+            if (type) HIPCK(h, hipMemcpyAsync(type, dtype, 4 * n, hipMemcpyDeviceToHost, h->stream));
+        }
+        HIPCK(h, hipStreamSynchronize(h->stream));
+        if (stage && xyz) memcpy(xyz, stage, 12 * n);
+        if (stage && type) memcpy(type, stage + 12 * n, 4 * n);
+        return RD_OK;
     }
     HIPCK(h, hipStreamSynchronize(h->stream));
-    if (xyz) memcpy(xyz, h->hxyz.data(), sizeof(float) * 3 * h->n);
-    if (type) memcpy(type, h->htype.data(), sizeof(int) * h->n);
     return RD_OK;
 }
 
@@ -1813,25 +1934,27 @@ extern "C" int rd_gradients(rd_system* h, float* grad, double* energy)
     int rc = refresh(h);
     if (rc) return rc;
     if (h->n == 0) { if (energy) *energy = 0.0; return RD_OK; }
-    HIPCK(h, hipMemsetAsync(h->d_etot, 0, sizeof(double), h->stream));
+    double* const d_etot = (double*)((char*)h->d_st + offsetof(RdStepState, etot));
+    HIPCK(h, hipMemsetAsync(d_etot, 0, sizeof(double), h->stream));
     if (h->ext_active()) rd_host_launch_ext(h);
     if (h->nwaves <= 3 * h->ncu)     // the line of lanes_per_particle
         hipLaunchKernelGGL((k_gradients_spread<9>), dim3(std::max(1, h->nwaves)), dim3(64 * 9), 0, h->stream, h->d_ps,
-                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, h->d_etot,
+                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, d_etot,
                            h->d_st);
     else
         hipLaunchKernelGGL(k_gradients, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_start, h->d_P,
-                           h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, h->d_etot, h->d_st);
+                           h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, d_etot, h->d_st);
     HIPCK(h, hipGetLastError());
-    std::vector<float> tmp(3 * (size_t)h->n);
-    double e = 0.0;
+    const size_t bytes = grad ? sizeof(float) * 3 * (size_t)h->n : 0;
     RdStepState st;
-    HIPCK(h, hipMemcpyAsync(tmp.data(), h->d_xyz_io, sizeof(float) * 3 * h->n, hipMemcpyDeviceToHost, h->stream));
-    HIPCK(h, hipMemcpyAsync(&e, h->d_etot, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCK(h, hipMemcpyAsync(&st, h->d_st, sizeof(st), hipMemcpyDeviceToHost, h->stream));
-    HIPCK(h, hipStreamSynchronize(h->stream));
-    if (grad) memcpy(grad, tmp.data(), sizeof(float) * 3 * h->n);
-    if (energy) *energy = e;
+    char* stage = rd_host_stage(h, sizeof(st) + bytes);
+    if (bytes)
+        HIPCK(h, hipMemcpyAsync(stage ? (void*)(stage + sizeof(st)) : (void*)grad, h->d_xyz_io, bytes,
+                                hipMemcpyDeviceToHost, h->stream));
+    rc = read_state(h, &st);
+    if (rc) return rc;
+    if (stage && bytes) memcpy(grad, stage + sizeof(st), bytes);
+    if (energy) *energy = st.etot;
     return (st.err & RD_ERR_FIXRANGE) ? step_error(h, RD_ERR_FIXRANGE) : RD_OK;
 }
 
@@ -2078,30 +2201,51 @@ static int pairs_common(rd_system* h, bool reactions, int64_t* out, long cap, lo
     uint32_t* d_off = h->d_poff;
     uint32_t* d_bs = h->d_pbs;
     uint32_t total = 0;
-    if (e == hipSuccess) launch_pair_counts(h, dtable, S, d_off, d_bs, h->d_pkeep);
-    if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&total, d_off + n, sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream);
+    char* stage = rd_host_stage(h, 64);
+    auto emit = [&]() {
+        hipLaunchKernelGGL((k_pairs_emit<uint2>), dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps,
+                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, dtable, S, d_off,
+                           (const uint32_t*)h->d_pkeep, h->d_pairs, (uint32_t)std::min(h->pairs_cap, (size_t)0xffffffffu));
+    };
+    if (e == hipSuccess) {
+        // the list is emitted at once, into the buffer of earlier calls; only
+        // a set that outgrew it waits for the total first
+        launch_pair_counts(h, dtable, S, d_off, d_bs, h->d_pkeep);
+        if (h->pairs_cap > 0) emit();
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(stage ? (void*)stage : (void*)&total, d_off + n, sizeof(uint32_t), hipMemcpyDeviceToHost,
+                           h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess && stage) memcpy(&total, stage, sizeof(total));
     if (e == hipSuccess && total > h->pairs_cap) {
         if (h->d_pairs) (void)hipFree(h->d_pairs);
         h->d_pairs = nullptr;
         h->pairs_cap = 0;
-        e = hipMalloc(&h->d_pairs, sizeof(uint2) * total);
-        if (e == hipSuccess) h->pairs_cap = total;
+        const size_t want = (size_t)total + total / 4 + 1024;
+        e = hipMalloc(&h->d_pairs, sizeof(uint2) * want);
+        if (e == hipSuccess) {
+            h->pairs_cap = want;
+            emit();
+            e = hipGetLastError();
+        }
     }
     const long nout = std::min<long>((long)total, cap);
-    std::vector<uint2> raw((size_t)nout);
-    if (e == hipSuccess && total > 0) {
-        hipLaunchKernelGGL((k_pairs_emit<uint2>), dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps,
-                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, dtable, S, d_off,
-                           (const uint32_t*)h->d_pkeep, h->d_pairs);
-        e = hipGetLastError();
-        if (e == hipSuccess && nout > 0)
-            e = hipMemcpyAsync(raw.data(), h->d_pairs, sizeof(uint2) * (size_t)nout, hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess && nout > 0) {
+        const size_t bytes = sizeof(uint2) * (size_t)nout;
+        std::vector<uint2> pageable;
+        uint2* raw = (uint2*)rd_host_stage(h, bytes);
+        if (!raw) {
+            pageable.resize((size_t)nout);
+            raw = pageable.data();
+        }
+        e = hipMemcpyAsync(raw, h->d_pairs, bytes, hipMemcpyDeviceToHost, h->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e == hipSuccess)
+            for (long k = 0; k < nout; ++k) { out[2 * k] = (int64_t)raw[k].x; out[2 * k + 1] = (int64_t)raw[k].y; }
     }
     if (e != hipSuccess) return set_err(h, RD_EHIP, std::string("pair emission: ") + hipGetErrorString(e));
-    for (long k = 0; k < nout; ++k) { out[2 * k] = (int64_t)raw[k].x; out[2 * k + 1] = (int64_t)raw[k].y; }
     if (count) *count = (long)total;
     return RD_OK;
 }
@@ -2172,7 +2316,7 @@ extern "C" int rd_reaction_candidates_noalloc(rd_system* h, int64_t* out, long c
     if (total > 0) {
         hipLaunchKernelGGL((k_pairs_emit<longlong2>), dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps,
                            h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, dtable, S, off,
-                           (const uint32_t*)nullptr, pairs);
+                           (const uint32_t*)nullptr, pairs, (uint32_t)RD_NA_MAX_PAIRS);
         HIPCK(h, hipGetLastError());
         const long nout = std::min<long>((long)total, cap);
         if (nout > 0)
@@ -2275,37 +2419,50 @@ static int apply_reactions(rd_system* h, const float* cr, const int* creation_re
         bty[k] = b.type;
         bxyz[3 * k] = b.x; bxyz[3 * k + 1] = b.y; bxyz[3 * k + 2] = b.z;
     }
-    int *d_del = nullptr, *d_shift = nullptr, *d_bdst = nullptr, *d_bty = nullptr;
-    float* d_bxyz = nullptr;
-    uint32_t* d_delcnt = nullptr;
+    // the lists in one buffer (all entries are 4 bytes), one copy to the device
     std::vector<uint32_t> delcnt((size_t)R * nt, 0);
-    hipError_t e = hipSuccess;
-    auto up = [&](auto** dst, const auto* src, size_t cnt) {
-        if (e != hipSuccess || cnt == 0) return;
-        e = hipMalloc((void**)dst, sizeof(**dst) * cnt);
-        if (e == hipSuccess) e = hipMemcpyAsync(*dst, src, sizeof(**dst) * cnt, hipMemcpyHostToDevice, h->stream);
+    const size_t words = del.size() + (size_t)R + 5 * born.size() + delcnt.size();
+    if (4 * words > h->react_cap) {
+        if (h->d_react) (void)hipFree(h->d_react);
+        h->d_react = nullptr;
+        h->react_cap = 0;
+        HIPCK(h, hipMalloc(&h->d_react, 8 * words));
+        h->react_cap = 8 * words;
+    }
+    std::vector<char> pageable;
+    char* lists = rd_host_stage(h, 4 * words);
+    if (!lists) {
+        pageable.resize(4 * words);
+        lists = pageable.data();
+    }
+    size_t at = 0;
+    auto put = [&](const void* src, size_t count) {
+        char* dst = h->d_react + at;
+        if (count) memcpy(lists + at, src, 4 * count);
+        at += 4 * count;
+        return (void*)dst;
     };
-    up(&d_del, del.data(), del.size());
-    up(&d_shift, shift.data(), (size_t)R);
-    up(&d_bdst, bdst.data(), bdst.size());
-    up(&d_bty, bty.data(), bty.size());
-    up(&d_bxyz, bxyz.data(), bxyz.size());
-    up(&d_delcnt, delcnt.data(), delcnt.size());
+    const uint32_t* d_delcnt = (const uint32_t*)put(delcnt.data(), delcnt.size());
+    const int* d_del = (const int*)put(del.data(), del.size());
+    const int* d_shift = (const int*)put(shift.data(), (size_t)R);
+    const int* d_bdst = (const int*)put(bdst.data(), bdst.size());
+    const int* d_bty = (const int*)put(bty.data(), bty.size());
+    const float* d_bxyz = (const float*)put(bxyz.data(), bxyz.size());
+    hipError_t e = hipMemcpyAsync(h->d_react, lists, 4 * words, hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess && n > 0)
         hipLaunchKernelGGL(k_react_compact, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_reps,
-                           h->d_waves, h->nwaves, d_del, (int)del.size(), d_shift, nt, d_delcnt, h->d_xyz_io,
+                           h->d_waves, h->nwaves, d_del, (int)del.size(), d_shift, nt, (uint32_t*)d_delcnt, h->d_xyz_io,
                            h->d_type_io);
     if (e == hipSuccess && !born.empty())
         hipLaunchKernelGGL(k_react_place, dim3(nblk((long)born.size(), RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream,
                            d_bxyz, d_bty, d_bdst, (int)born.size(), h->d_xyz_io, h->d_type_io);
     if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess && d_delcnt)
-        e = hipMemcpyAsync(delcnt.data(), d_delcnt, sizeof(uint32_t) * delcnt.size(), hipMemcpyDeviceToHost, h->stream);
-    hipError_t se = hipStreamSynchronize(h->stream);
-    for (void* p : { (void*)d_del, (void*)d_shift, (void*)d_bdst, (void*)d_bty, (void*)d_bxyz, (void*)d_delcnt })
-        if (p) (void)hipFree(p);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(lists, d_delcnt, sizeof(uint32_t) * delcnt.size(), hipMemcpyDeviceToHost, h->stream);
+    const hipError_t se = hipStreamSynchronize(h->stream);
     if (e != hipSuccess || se != hipSuccess)
         return set_err(h, RD_EHIP, std::string("reaction compaction: ") + hipGetErrorString(e != hipSuccess ? e : se));
+    memcpy(delcnt.data(), lists, sizeof(uint32_t) * delcnt.size());
     // particle counts per (replica, type); the host position/type mirrors are
     // refreshed from the device when next read
     for (size_t k = 0; k < delcnt.size(); ++k) h->tcount[k] -= (long)delcnt[k];
