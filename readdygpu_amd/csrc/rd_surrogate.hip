@@ -952,30 +952,36 @@ __global__ __launch_bounds__(256) void k_mlp_slots(const RdMlpPack* __restrict__
                                                    float4* __restrict__ gext)
 {
     __shared__ RdMlpFwdLds L;
-    __shared__ uint32_t ring[4][RD_MLP_RING];
+    __shared__ float4 ring[4][RD_MLP_RING];              // normalised position, slot
     mlp_stage<256>(L, pk);
     __syncthreads();
     const int lane = threadIdx.x & 63, j = lane & 15;
-    uint32_t* q = ring[threadIdx.x >> 6];
+    float4* q = ring[threadIdx.x >> 6];
     auto tile = [&](uint32_t head, int cnt) {            // cnt in 1..16 entries from head
         const bool ok = j < cnt;
-        const uint32_t s = ok ? q[(head + j) & (RD_MLP_RING - 1)] : 0u;
-        const float4 p = ps[s];
-        float xn[3] = { norm_coord(p.x, nm.lo[0], nm.sc[0]), norm_coord(p.y, nm.lo[1], nm.sc[1]),
-                        norm_coord(p.z, nm.lo[2], nm.sc[2]) };
+        const float4 p = q[(head + (ok ? j : 0)) & (RD_MLP_RING - 1)];
+        const float xn[3] = { p.x, p.y, p.z };
         const float3 y = mlp_tile(L, xn);
         if (lane < 16 && ok)
-            gext[s] = make_float4(y.x * nm.gscale, y.y * nm.gscale, y.z * nm.gscale, 0.f);
+            gext[__float_as_uint(p.w)] = make_float4(y.x * nm.gscale, y.y * nm.gscale, y.z * nm.gscale, 0.f);
     };
     const long nchunks = ((long)n + 63) / 64;
     const long wpb = blockDim.x >> 6;
     const long stride = (long)gridDim.x * wpb;
     uint32_t head = 0, tail = 0;                         // tail - head <= 15 between chunks
-    for (long c = (long)xcd_block(blockIdx.x, gridDim.x) * wpb + (threadIdx.x >> 6); c < nchunks; c += stride) {
+    long c = (long)xcd_block(blockIdx.x, gridDim.x) * wpb + (threadIdx.x >> 6);
+    float4 next = make_float4(0.f, 0.f, 0.f, 0.f);       // the next chunk's record, a chunk ahead
+    if (c * 64 + lane < n) next = ps[c * 64 + lane];
+    for (; c < nchunks; c += stride) {
         const long s = c * 64 + lane;
-        const bool on = s < n && ((type_mask >> w_type(ps[s].w)) & 1u);
+        const float4 p = next;
+        if (s + stride * 64 < n) next = ps[s + stride * 64];
+        const bool on = s < n && ((type_mask >> w_type(p.w)) & 1u);
         const uint64_t b = __ballot(on);
-        if (on) q[(tail + lanes_below(b)) & (RD_MLP_RING - 1)] = (uint32_t)s;
+        if (on)
+            q[(tail + lanes_below(b)) & (RD_MLP_RING - 1)] =
+                make_float4(norm_coord(p.x, nm.lo[0], nm.sc[0]), norm_coord(p.y, nm.lo[1], nm.sc[1]),
+                            norm_coord(p.z, nm.lo[2], nm.sc[2]), __uint_as_float((uint32_t)s));
         tail += (uint32_t)__popcll(b);
         wave_lds_sync();
 #pragma unroll 1
