@@ -45,6 +45,7 @@ struct rd_system {
     std::vector<RdWave> wave_tab;
     std::vector<long> tcount;        // particles per (replica, type), [R * nt]
     int nwaves = 0;
+    bool queue_form = false;         // the step's force kernel deals the hits out (gather_queue)
 
     // particles in index order (host mirror)
     int n = 0;

@@ -295,26 +295,44 @@ struct RdAcc {
     bool sat;
 };
 
-// s += floor(v * 2^32), clamped to the range: the integer part and the exact
+// floor(v * 2^32), clamped to the range: the integer part and the exact
 // fraction from two 32-bit conversions (instead of a float -> int64
-// conversion sequence), added as the low word and, with its carry, the high
-// word
-__device__ __forceinline__ void fix_add(long long& s, float v)
+// conversion sequence) as the high and low words
+__device__ __forceinline__ void fix_words(float v, uint32_t& hi, uint32_t& lo)
 {
     v = fminf(fmaxf(v, -RD_FIX_MAX), RD_FIX_MAX);
     const float fl = floorf(v);
-    const uint32_t hi = (uint32_t)(int)fl;
-    const uint32_t lo = (uint32_t)((v - fl) * RD_FIX_SCALE);
+    hi = (uint32_t)(int)fl;
+    lo = (uint32_t)((v - fl) * RD_FIX_SCALE);
+}
+
+__device__ __forceinline__ unsigned long long fix_term(float v)
+{
+    uint32_t hi, lo;
+    fix_words(v, hi, lo);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// s += that, as the low word and, with its carry, the high word
+__device__ __forceinline__ void fix_add(long long& s, float v)
+{
+    uint32_t hi, lo;
+    fix_words(v, hi, lo);
     unsigned int c;
     const uint32_t sl = __builtin_addc((uint32_t)s, lo, 0u, &c);
     const uint32_t sh = __builtin_addc((uint32_t)((unsigned long long)s >> 32), hi, c, &c);
     s = (long long)(((unsigned long long)sh << 32) | sl);
 }
 
+__device__ __forceinline__ bool fix_range(float fx, float fy, float fz)
+{
+    return fabsf(fx) < RD_FIX_MAX && fabsf(fy) < RD_FIX_MAX && fabsf(fz) < RD_FIX_MAX;
+}
+
 __device__ __forceinline__ void acc_add(RdAcc& a, float pre, float dx, float dy, float dz)
 {
     const float fx = pre * dx, fy = pre * dy, fz = pre * dz;
-    a.sat = a.sat || !(fabsf(fx) < RD_FIX_MAX && fabsf(fy) < RD_FIX_MAX && fabsf(fz) < RD_FIX_MAX);
+    a.sat = a.sat || !fix_range(fx, fy, fz);
     fix_add(a.x, fx); fix_add(a.y, fy); fix_add(a.z, fz);
 }
 
@@ -474,10 +492,12 @@ __device__ __forceinline__ void bond_accum(const RdDev* __restrict__ P, const Rd
 }
 
 // per-wave list of candidate pairs that passed the distance test (slot of
-// the partner), transposed so that a wave's lanes write one LDS row
-#define RD_HITS 16
+// the partner), transposed so that a wave's lanes write one LDS row: RD_HITS
+// listed hits, then a row for the first hit past them and one for the rest
+// (written without a branch, 3 instructions a hit instead of 8)
+#define RD_HITS 14
 struct RdHitList {
-    uint32_t j[RD_HITS][64];
+    uint32_t j[RD_HITS + 2][64];
 };
 
 // gradient of U (pair + external) for the particle in slot s, from global
@@ -532,7 +552,7 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
             // whose six bounds are loaded together (independent loads in
             // flight at once).
             // Dense stencils: a lane whose list fills notes its first
-            // unlisted hit (run, slot) and stops listing; before its next
+            // unlisted hit (its slot) and stops listing; before its next
             // run the wave leaves the listing-only walk for a second one
             // that goes on from there, listing while a lane's list has room
             // and evaluating further hits as they are met.  Keeping the
@@ -540,9 +560,7 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
             // registers free (inlined there, it made the compiler reload the
             // particle array's address from the kernel arguments on every
             // iteration).
-            int nhit = 0;                   // hits met; more than RD_HITS: the list is full
-            int cur_run = 0, res_run = 0;   // (res_run, res_j): the first unlisted hit
-            uint32_t res_j = 0u;
+            uint32_t nhit = 0;              // hits met; more than RD_HITS: the list is full
             auto delta = [&](float4 q, float& dx, float& dy, float& dz) {
                 dx = p.x - q.x; dy = p.y - q.y; dz = p.z - q.z;
                 if (!in) {
@@ -567,10 +585,7 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                 }
                 const float d2 = dist2(dx, dy, dz);
                 if (d2 < T.rc2[rowbase + w_type(q.w)] && d2 > 0.0f) {
-                    if (nhit < RD_HITS) il->j[nhit][lane] = j;
-                    const bool first = nhit == RD_HITS;
-                    res_j = first ? j : res_j;
-                    res_run = first ? cur_run : res_run;
+                    il->j[min(nhit, RD_HITS + 1u)][lane] = j;
                     ++nhit;
                 }
             };
@@ -650,7 +665,6 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                                 stop = true;
                                 rnext = g + k;
                             } else {
-                                cur_run = g + k;
                                 walk(sb[k], se[k]);
                             }
                         }
@@ -658,11 +672,13 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                 }
             }
             const bool over = nhit > RD_HITS;
-            nhit = min(nhit, RD_HITS);
+            nhit = min(nhit, (uint32_t)RD_HITS);
             if (__any(over)) {
                 // go on from the run in which lists filled (rnext - 1, the
-                // last one walked): lanes whose list filled from their first
-                // unlisted hit, the others from run rnext
+                // last one walked, as the wave stops before the next): lanes
+                // whose list filled from their first unlisted hit, the others
+                // from run rnext
+                const uint32_t res_j = il->j[RD_HITS][lane];
 #pragma unroll 1
                 for (int r0 = rnext - 1; r0 < nruns; r0 += 3) {
                     uint32_t sb[3], se[3];
@@ -671,9 +687,9 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                         const int run = r0 + r;
                         sb[r] = 0u;
                         se[r] = 0u;
-                        if (run < nruns && run >= (over ? res_run : rnext)) {
+                        if (run < nruns && run >= (over ? rnext - 1 : rnext)) {
                             bounds(run, sb[r], se[r]);
-                            if (over && run == res_run) sb[r] = res_j;
+                            if (over && run == rnext - 1) sb[r] = res_j;
                         }
                     }
 #pragma unroll
@@ -693,7 +709,7 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
             if (__any(nhit > 0)) {
                 float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (nhit > 0) q = pv(il->j[0][lane]);
-                for (int k = 0; __any(k < nhit); ++k) {
+                for (uint32_t k = 0; __any(k < nhit); ++k) {
                     float4 n = q;
                     if (k + 1 < nhit) n = pv(il->j[k + 1][lane]);
                     if (k < nhit) {
@@ -716,6 +732,184 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
     if (ENERGY) *energy = e;
     *sat = acc.sat;
     return g;
+}
+
+// ---- a wave's hits in one queue ----
+// A wave's LDS: the queue of candidate pairs that passed the distance test
+// (home lane in the top 6 bits, slot of the partner below: slots are below
+// 2^26), the homes' records and the homes' fixed-point sums.
+#define RD_QUEUE 384
+struct RdWaveLds {
+    uint32_t q[RD_QUEUE];
+    float4 home[64];
+    unsigned long long f[3][64];
+};
+
+// Pair terms of the wave's particles, added to wl->f (the caller has stored
+// the homes and cleared the sums); every lane of the wave calls it (`act`: the
+// lane holds a particle).  Returns whether a term the lane evaluated left the
+// fixed-point range.  Needs S = 1 and at least three cells per axis.  The same
+// pairs, terms and integer sums as gather_grad, so the same bits, but:
+// - the wave's hits go to one queue, whichever lane met them, and are dealt to
+//   the 64 lanes for evaluation, which adds a pair's term to its home's sums in
+//   LDS (integers: the order does not matter).  With each lane evaluating its
+//   own hits, the interaction code runs as often as the lane with the most hits
+//   needs (vector instructions bound this kernel: 91% busy in the cytosol), and
+//   a lane with more than its list holds sends the wave into a second walk;
+// - a row's two runs are walked as one sequence per lane, so that a wave
+//   iterates over the largest sum of a lane's runs, not over the largest first
+//   run and then the largest second one (16 to 19% fewer slots in lattices of
+//   12 to 41 cells);
+// - every test takes the minimum image's magnitudes, without a branch.
+// Which of the two forms a step takes: queue_form_pays.
+__device__ __forceinline__ bool gather_queue(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
+                                             const float4* __restrict__ ps, const uint32_t* __restrict__ start, float4 p,
+                                             bool act, RdWaveLds* __restrict__ wl)
+{
+    const int rowbase = w_type(p.w) * P->nt, lane = threadIdx.x & 63;
+    const int Lx = R.L[0], Ly = R.L[1], Lz = R.L[2];
+    int cx, cy, cz;
+    cell_coords(R, p.x, p.y, p.z, cx, cy, cz);
+    // the particle array's address in vector registers, as in gather_grad
+    typedef float rd_f4 __attribute__((ext_vector_type(4)));
+    typedef const __attribute__((address_space(1))) rd_f4* gptr;
+    gptr pva;
+    {
+        const uint64_t a = (uint64_t)(uintptr_t)ps;
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(lane << 2, (int)(uint32_t)a);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(lane << 2, (int)(uint32_t)(a >> 32));
+        pva = (gptr)(((uint64_t)hi << 32) | lo);
+    }
+    uint32_t qn = 0;                // queued pairs (the same in every lane)
+    bool sat = false;
+    const uint32_t tag = (uint32_t)lane << 26;
+    auto flush = [&](uint32_t cnt) {
+        wave_lds_sync();
+        for (uint32_t b = 0; b < cnt; b += 64) {
+            if (b + (uint32_t)lane >= cnt) continue;
+            const uint32_t e = wl->q[b + lane], hl = e >> 26;
+            const rd_f4 q = pva[e & 0x3ffffffu];
+            const float4 h = wl->home[hl];
+            const float dx = min_image(h.x - q.x, R.Lb[0], R.half[0]);
+            const float dy = min_image(h.y - q.y, R.Lb[1], R.half[1]);
+            const float dz = min_image(h.z - q.z, R.Lb[2], R.half[2]);
+            const float d2 = dist2(dx, dy, dz);
+            const int pair = w_type(h.w) * P->nt + w_type(q.w);
+            const float rinv = __builtin_amdgcn_rsqf(d2);
+            float ep = 0.0f;
+            const float pre = pair_pre_wave<false>(T.pot2, T.npot, T.mask[pair], T.r0[pair], d2 * rinv, rinv, &ep);
+            const float fx = pre * dx, fy = pre * dy, fz = pre * dz;
+            sat = sat || !fix_range(fx, fy, fz);
+            atomicAdd(&wl->f[0][hl], fix_term(fx));
+            atomicAdd(&wl->f[1][hl], fix_term(fy));
+            atomicAdd(&wl->f[2][hl], fix_term(fz));
+        }
+        wave_lds_sync();
+    };
+    // `full`: hits were left out because the queue has no room for 64 more
+    auto test = [&](bool valid, uint32_t j, rd_f4 q, bool& full) {
+        const float d2 = dist2(min_image_abs(p.x - q.x, R.Lb[0]), min_image_abs(p.y - q.y, R.Lb[1]),
+                               min_image_abs(p.z - q.z, R.Lb[2]));
+        const uint64_t m = __builtin_amdgcn_ballot_w64(valid & (d2 < T.rc2[rowbase + w_type(q.w)]) & (d2 > 0.0f));
+        if (m) {
+            if (qn <= RD_QUEUE - 64) {
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) wl->q[qn + (uint32_t)lanes_below(m)] = tag | j;
+                qn += (uint32_t)__popcll(m);
+            } else {
+                full = true;
+            }
+        }
+    };
+    int a0, b0, a1 = 0, b1 = -1;
+    const int nr = x_runs(cx, 1, Lx, &a0, &b0, &a1, &b1);
+    // bounds of row r's first and second run (empty for lanes without one);
+    // both from one 16-byte load, as in gather_grad
+    auto bounds = [&](int r, uint32_t& j, uint32_t& e, uint32_t& j2, uint32_t& e2) {
+        j = e = j2 = e2 = 0u;
+        int yy = cy + (r % 3) - 1, zz = cz + (r / 3) - 1;
+        yy += yy < 0 ? Ly : 0; yy -= yy >= Ly ? Ly : 0;
+        zz += zz < 0 ? Lz : 0; zz -= zz >= Lz ? Lz : 0;
+        const uint32_t* row = start + R.coff + (zz * Ly + yy) * Lx;
+        uint4 v;
+        if (act) {
+            __builtin_memcpy(&v, row + a0, sizeof(v));
+            const int len = b0 + 1 - a0;
+            j = v.x;
+            e = len == 3 ? v.w : (len == 2 ? v.z : v.y);
+            if (nr == 2) {
+                __builtin_memcpy(&v, row + a1, sizeof(v));
+                j2 = v.x;
+                e2 = b1 + 1 - a1 == 2 ? v.z : v.y;
+            }
+        }
+    };
+    // slots j .. e-1, then j2 .. e2-1, two at a time, the next two loaded while
+    // the current two are tested.  The whole wave goes on until its last lane
+    // is done (the queue's count stays the same in every lane); the loads may
+    // read the record after a run (the array has 16 records of padding).
+    auto walk = [&](uint32_t j, uint32_t e, uint32_t j2, uint32_t e2, bool& full) {
+        const bool skip = j >= e;
+        j = skip ? j2 : j; e = skip ? e2 : e; e2 = skip ? 0u : e2;
+        if (!__any(j < e)) return;
+        rd_f4 q0 = {}, q1 = {};
+        if (j < e) { gptr a = pva + j; q0 = a[0]; q1 = a[1]; }
+        do {
+            const bool next = j + 2 >= e;
+            const uint32_t jn = next ? j2 : j + 2, en = next ? e2 : e;
+            e2 = next ? 0u : e2;
+            rd_f4 n0 = q0, n1 = q1;
+            if (jn < en) { gptr a = pva + jn; n0 = a[0]; n1 = a[1]; }
+            test(j < e, j, q0, full);
+            test(j + 1 < e, j + 1, q1, full);
+            j = jn; e = en;
+            q0 = n0; q1 = n1;
+        } while (__any(j < e));
+    };
+    // A row whose hits do not fit is taken out of the queue again, and the
+    // wave leaves the unrolled walk for a second one that starts at this row
+    // and evaluates the queue whenever it is nearly full.
+    int rnext = 9;
+    bool stop = false;
+#pragma unroll
+    for (int g = 0; g < 9; g += 3) {
+        if (!stop) {
+            uint32_t sb[3], se[3], tb[3], te[3];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) bounds(g + r, sb[r], se[r], tb[r], te[r]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (!stop) {
+                    const uint32_t before = qn;
+                    walk(sb[k], se[k], tb[k], te[k], stop);
+                    if (stop) {
+                        qn = before;
+                        rnext = g + k;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll 1
+    for (int r = rnext; r < 9; ++r) {
+        uint32_t j, e, j2, e2;
+        bounds(r, j, e, j2, e2);
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll 1
+            while (__any(j < e)) {
+                if (qn > RD_QUEUE - 128) { flush(qn); qn = 0; }
+                rd_f4 q0 = {}, q1 = {};
+                if (j < e) { q0 = pva[j]; q1 = pva[j + 1]; }
+                bool never = false;
+                test(j < e, j, q0, never);
+                test(j + 1 < e, j + 1, q1, never);
+                j += 2;
+            }
+            j = j2; e = e2;
+        }
+    }
+    flush(qn);
+    return sat;
 }
 
 // Pair and bond terms of the particle in slot s shared by G lanes (sub = 0 ..

@@ -102,6 +102,36 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void
     force_update<BLOCK, 1>(ps, pn, kr, count, tsum, start, P, reps, waves, nwaves, pot1, st, noise, ntot);
 }
 
+// One particle per lane, the wave's hits in one queue (gather_queue)
+__global__ __launch_bounds__(RD_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_force_update_dealt(RD_FORCE_ARGS)
+{
+    __shared__ RdTab T;
+    __shared__ RdWaveLds wl[RD_BLOCK / 64];
+    const int lane = threadIdx.x & 63;
+    const RdWave it = wave_item(waves, nwaves, __builtin_amdgcn_readfirstlane(wave_id()));
+    const uint32_t s = (uint32_t)(it.s0 + lane);
+    const bool act = s < (uint32_t)it.s1;
+    float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (act) p = ps[s];
+    RdWaveLds& w = wl[threadIdx.x >> 6];
+    w.home[lane] = p;
+    w.f[0][lane] = 0ull; w.f[1][lane] = 0ull; w.f[2][lane] = 0ull;
+    load_tab<RD_BLOCK>(T, P);
+    if (it.s0 >= it.s1) return;
+    const RdRep R = reps[it.rep];
+    RdAcc acc;
+    acc.e = 0.0;
+    acc.sat = gather_queue(P, R, T, ps, start, p, act, &w);
+    if (acc.sat && !act) atomicOr(&st->err, RD_ERR_FIXRANGE);   // (another lane's pair)
+    if (!act) return;
+    acc.x = (long long)w.f[0][lane];
+    acc.y = (long long)w.f[1][lane];
+    acc.z = (long long)w.f[2][lane];
+    if (P->bstart) bond_accum<false>(P, R, T, ps, p, acc);
+    const float3 g = finish_grad<false>(P, T, pot1, s, p, acc, nullptr);
+    em_update_store(P, R, T, st, s, p, g, step_noise(P, R, st, noise, ntot, w_index(p.w)), acc.sat, pn, kr, count, tsum);
+}
+
 // PPT > 1 particles per lane (the compiler's own register budget)
 template <int BLOCK, int PPT>
 __global__ __launch_bounds__(BLOCK) void k_force_update_ppt(RD_FORCE_ARGS)
@@ -1138,6 +1168,7 @@ extern "C" int rd_set_bonds(rd_system* h, int n_bonds, const int* bonds, const i
 {
     if (!h || n_bonds < 0 || n_pots < 0) return RD_EINVAL;
     if (n_bonds > 0 && (!bonds || !pot_index || n_pots == 0 || !pots)) return RD_EINVAL;
+    static_assert(RD_MAX_PARTICLES <= (1 << 26), "a slot takes 26 bits of a gather_queue entry");
     static_assert(RD_MAXBP == RD_MAX_BOND_POTS, "bond potential limits differ");
     if (n_pots > RD_MAXBP) return set_err(h, RD_EINVAL, "too many bond potentials (at most " + std::to_string(RD_MAXBP) + ")");
     for (int p = 0; p < n_pots; ++p) {
@@ -1174,6 +1205,32 @@ static double pair_range(const rd_system* h, int i, int j, double r0)
         m = std::max(m, std::min(r, h->prm.max_cutoff));
     }
     return m;
+}
+
+// Whether the step's force kernel takes the queue form (gather_queue) or the
+// list form (gather_grad).  The queue's fixed cost (homes and sums in LDS, the
+// run switch in every iteration) is paid back by the hits it deals out, so the
+// rule is the expected number of partners in range of a particle: density times
+// the mean volume of a pair's range over the type pairs.  Measured, list ->
+// queue form, us a step at 0.6M particles, two species, lattices of 12 / 48 /
+// 128 cells along x:
+//   0.15 partners: 86 -> 86 / 87 -> 91 / 80 -> 84
+//   0.38 partners: 64 -> 60 / 65 -> 63 / 64 -> 63
+//   1.1 partners:  64 -> 58 / 67 -> 64 / 75 -> 76
+//   3.8 partners:  86 -> 75 / 92 -> 87 / 266 -> 249 (2.9M)
+// and 1M particles in four species (0.32 partners, 165 cells) 96.0 -> 98.3, the
+// 16 crowded cytosol boxes (2.1 partners) 179 -> 159, after 600 steps 485 -> 402.
+static bool queue_form_pays(const RdDev& P, const std::vector<RdRep>& reps)
+{
+    if (P.S != 1 || !P.n_pot2) return false;    // the walk is of the nearest cells
+    double n = 0.0, vol = 0.0, rc3 = 0.0;
+    for (const RdRep& R : reps) {
+        if (R.L[0] < 3 || R.L[1] < 3 || R.L[2] < 3) return false;   // a cell may not be met twice
+        n += R.n;
+        vol += (double)R.Lb[0] * R.Lb[1] * R.Lb[2];
+    }
+    for (int k = 0; k < P.nt * P.nt; ++k) rc3 += std::pow((double)P.rc2[k], 1.5);
+    return n * (4.0 / 3.0 * M_PI) * rc3 / ((double)P.nt * P.nt) >= 0.35 * vol;
 }
 
 double rd_host_r0(const rd_system* h, int i, int j)
@@ -1286,6 +1343,7 @@ static int build_tables(rd_system* h)
             wave_tab.push_back(w);
         }
     }
+    h->queue_form = queue_form_pays(P, rep_dev);
     h->P = P;
     h->max_range = maxr;
     h->max_rxn = maxrx;
@@ -1386,7 +1444,7 @@ static int grow_particles(rd_system* h, int need, bool keep_ps)
     drop_graph(h);
     int cap = std::max(need, h->cap + h->cap / 2);
     float4* nps = nullptr;
-    HIPCK(h, hipMalloc(&nps, sizeof(float4) * cap));
+    HIPCK(h, hipMalloc(&nps, sizeof(float4) * ((size_t)cap + 16)));     // the walks load the record after a run
     if (keep_ps && h->d_ps && h->n > 0) {
         HIPCK(h, hipMemcpyAsync(nps, h->d_ps, sizeof(float4) * (size_t)h->n, hipMemcpyDeviceToDevice, h->stream));
         HIPCK(h, hipStreamSynchronize(h->stream));
@@ -1592,6 +1650,20 @@ static void launch_force_ppt(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 void rd_host_launch_force(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 {
     if (h->n <= 0) return;
+    if (h->kern == RD_KERNEL_GATHER && h->block == 256 && h->ppt == 1 && lanes_per_particle(h) == 1 && h->queue_form) {
+        const dim3 grid(wave_blocks(h));
+        if (ev0)
+            hipExtLaunchKernelGGL(k_force_update_dealt, grid, dim3(RD_BLOCK), 0, h->stream, ev0, ev1, 0,
+                                  (const float4*)h->d_ps, h->d_pn, h->d_kr, h->d_count, h->d_bsum,
+                                  (const uint32_t*)h->d_start, (const RdDev*)h->d_P, (const RdRep*)h->d_reps,
+                                  (const RdWave*)h->d_waves, h->nwaves, (const RdPot1Dev*)h->d_pot1, h->d_st,
+                                  (const float*)h->d_noise, h->n);
+        else
+            hipLaunchKernelGGL(k_force_update_dealt, grid, dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_pn, h->d_kr,
+                               h->d_count, h->d_bsum, h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1,
+                               h->d_st, h->d_noise, h->n);
+        return;
+    }
     switch (lanes_per_particle(h)) {
     case 9: launch_force_spread<9>(h, ev0, ev1); return;
     case 3: launch_force_spread<3>(h, ev0, ev1); return;
