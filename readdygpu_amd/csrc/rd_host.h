@@ -14,6 +14,9 @@
 
 struct RdStepState;
 
+// forms of the force kernel's gather (force_form in rd_system.hip)
+enum { RD_FORM_ROWS, RD_FORM_SPARSE, RD_FORM_DEALT };
+
 struct rd_system {
     rd_params prm{};
     std::string err;
@@ -45,7 +48,8 @@ struct rd_system {
     std::vector<RdWave> wave_tab;
     std::vector<long> tcount;        // particles per (replica, type), [R * nt]
     int nwaves = 0;
-    bool queue_form = false;         // the step's force kernel deals the hits out (gather_queue)
+    int force_form[2] = {};          // the step's force kernel at one particle per lane, without
+                                     // and with an external pass (RD_FORM_*)
 
     // particles in index order (host mirror)
     int n = 0;

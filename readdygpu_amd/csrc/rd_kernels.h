@@ -501,8 +501,9 @@ struct RdHitList {
 };
 
 // gradient of U (pair + external) for the particle in slot s, from global
-// memory (the per-particle gather)
-template <bool ENERGY>
+// memory (the per-particle gather).  SPARSE: candidates are listed before they
+// are tested (force_form says when)
+template <bool ENERGY, bool SPARSE = false>
 __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
                                               const RdPot1Dev* __restrict__ pot1,
                                               const float4* __restrict__ ps, const uint32_t* __restrict__ start,
@@ -650,8 +651,86 @@ __device__ __forceinline__ float3 gather_grad(const RdDev* __restrict__ P, const
                 }
                 if (j < j1) test(j, pv(j));
             };
+            // SPARSE: all candidates of a lane first go to its list (their
+            // slots, from the rows' bounds), and are tested from there, four
+            // loads in flight, the hits packed at the list's head.  A wave
+            // thus tests as often as its lane with the most candidates needs
+            // (2M particles, 2.2 candidates each: 8 to 9 times), where a walk
+            // by rows adds up every row's largest run (about 20).  A wave with
+            // more than `few` candidates in a lane, or a run of more than four
+            // slots, walks by rows instead.
+            bool listed = false;
+            if constexpr (SPARSE) {
+                constexpr uint32_t few = RD_HITS - 2;
+                uint32_t c = 0, most = 0;   // slots listed, longest run
+                // four slots are written and as many counted as the run has;
+                // the list's last rows take those of a list that is full
+                auto take = [&](uint32_t j, uint32_t e) {
+                    const uint32_t len = e - j;
+                    most = max(most, len);
+                    uint32_t(*l)[64] = il->j + min(c, few);
+                    l[0][lane] = j;
+                    l[1][lane] = j + 1;
+                    if (__any(len > 2)) {
+                        l[2][lane] = j + 2;
+                        l[3][lane] = j + 3;
+                    }
+                    c += len;
+                };
+                listed = true;
+#pragma unroll
+                for (int h = 0; h < 3; ++h) {
+                    const int g = h == 0 ? 3 : (h == 1 ? 0 : 6);    // the home's own layer first
+                    if (listed) {
+                        uint32_t sb[3], se[3];
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) bounds(g + r, sb[r], se[r]);
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) take(sb[r], se[r]);
+                        listed = !__any((c > few) | (most > 4));
+                    }
+                }
+                if (listed && nr == 2) {
+#pragma unroll
+                    for (int g = 9; g < 18; g += 3) {
+                        uint32_t sb[3], se[3];
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) bounds(g + r, sb[r], se[r]);
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) take(sb[r], se[r]);
+                    }
+                }
+                listed = !__any((c > few) | (most > 4));
+                if (listed) {
+#pragma unroll 1
+                    for (uint32_t k = 0; __any(k < c); k += 4) {
+                        uint32_t j[4];
+                        float4 q[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            j[i] = il->j[k + i][lane];
+                            j[i] = k + i < c ? j[i] : s;        // (its own slot: no hit)
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) q[i] = pv(j[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float d2 = dist2(min_image_abs(p.x - q[i].x, R.Lb[0]),
+                                                   min_image_abs(p.y - q[i].y, R.Lb[1]),
+                                                   min_image_abs(p.z - q[i].z, R.Lb[2]));
+                            if (d2 < T.rc2[rowbase + w_type(q[i].w)] && d2 > 0.0f) {
+                                il->j[nhit][lane] = j[i];
+                                ++nhit;
+                            }
+                        }
+                    }
+                }
+                // (the walk by rows takes its bounds anew: the compiler would
+                // else keep those of all rows, 20 registers more than there are)
+                asm volatile("" : "+v"(cy), "+v"(cz), "+v"(a0), "+v"(a1));
+            }
             int rnext = nruns;              // first run the listing-only walk did not reach
-            bool stop = false;
+            bool stop = listed;
 #pragma unroll
             for (int g = 0; g < 18; g += 3) {
                 if (g < nruns && !stop) {
@@ -761,7 +840,7 @@ struct RdWaveLds {
 //   run and then the largest second one (16 to 19% fewer slots in lattices of
 //   12 to 41 cells);
 // - every test takes the minimum image's magnitudes, without a branch.
-// Which of the two forms a step takes: queue_form_pays.
+// Which form a step takes: force_form.
 __device__ __forceinline__ bool gather_queue(const RdDev* __restrict__ P, const RdRep& R, const RdTab& T,
                                              const float4* __restrict__ ps, const uint32_t* __restrict__ start, float4 p,
                                              bool act, RdWaveLds* __restrict__ wl)

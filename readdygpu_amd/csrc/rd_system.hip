@@ -57,7 +57,7 @@ __device__ __forceinline__ int wave_id() { return xcd_block(blockIdx.x, gridDim.
         const RdDev *__restrict__ P, const RdRep *__restrict__ reps, const RdWave *__restrict__ waves, \
         int nwaves, const RdPot1Dev *__restrict__ pot1, RdStepState *__restrict__ st,                   \
         const float *__restrict__ noise, int ntot
-template <int BLOCK, int PPT>
+template <int BLOCK, int PPT, bool SPARSE = false>
 __device__ __forceinline__ void force_update(RD_FORCE_ARGS)
 {
     __shared__ RdTab T;
@@ -75,7 +75,8 @@ __device__ __forceinline__ void force_update(RD_FORCE_ARGS)
         if (!act) return;
         const RdRep R = reps[it.rep];
         bool sat;
-        float3 g = gather_grad<false>(P, R, T, pot1, ps, start, s, p, nullptr, &sat, &il[threadIdx.x >> 6]);
+        float3 g = gather_grad<false, SPARSE>(P, R, T, pot1, ps, start, s, p, nullptr, &sat,
+                                              &il[threadIdx.x >> 6]);
         em_update_store(P, R, T, st, s, p, g, step_noise(P, R, st, noise, ntot, w_index(p.w)), sat, pn, kr, count, tsum);
     } else {
         load_tab<BLOCK>(T, P);
@@ -100,6 +101,12 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_force_update(RD_FORCE_ARGS)
 {
     force_update<BLOCK, 1>(ps, pn, kr, count, tsum, start, P, reps, waves, nwaves, pot1, st, noise, ntot);
+}
+
+// The same, a particle's candidates listed before they are tested
+__global__ __launch_bounds__(RD_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_force_update_sparse(RD_FORCE_ARGS)
+{
+    force_update<RD_BLOCK, 1, true>(ps, pn, kr, count, tsum, start, P, reps, waves, nwaves, pot1, st, noise, ntot);
 }
 
 // One particle per lane, the wave's hits in one queue (gather_queue)
@@ -1207,30 +1214,40 @@ static double pair_range(const rd_system* h, int i, int j, double r0)
     return m;
 }
 
-// Whether the step's force kernel takes the queue form (gather_queue) or the
-// list form (gather_grad).  The queue's fixed cost (homes and sums in LDS, the
-// run switch in every iteration) is paid back by the hits it deals out, so the
-// rule is the expected number of partners in range of a particle: density times
-// the mean volume of a pair's range over the type pairs.  Measured, list ->
-// queue form, us a step at 0.6M particles, two species, lattices of 12 / 48 /
-// 128 cells along x:
-//   0.15 partners: 86 -> 86 / 87 -> 91 / 80 -> 84
-//   0.38 partners: 64 -> 60 / 65 -> 63 / 64 -> 63
-//   1.1 partners:  64 -> 58 / 67 -> 64 / 75 -> 76
-//   3.8 partners:  86 -> 75 / 92 -> 87 / 266 -> 249 (2.9M)
-// and 1M particles in four species (0.32 partners, 165 cells) 96.0 -> 98.3, the
-// 16 crowded cytosol boxes (2.1 partners) 179 -> 159, after 600 steps 485 -> 402.
-static bool queue_form_pays(const RdDev& P, const std::vector<RdRep>& reps)
+// Which form of the gather the step's force kernel takes (at one particle per
+// lane): candidates listed before they are tested (gather_grad, SPARSE) where
+// a particle has few, hits dealt out (gather_queue) where it expects partners
+// enough to pay for the queue's fixed cost (homes and sums in LDS, the run
+// switch in every iteration), else a walk by rows (gather_grad).  The rules are
+// 27 cells' mean occupancy and the expected number of partners in range, the
+// density times the mean volume of a pair's range over the type pairs.
+// Measured, rows / sparse / dealt, us a step at 0.6M particles of two species,
+// 12 and 64 cells along x:
+//   candidates 0.8, partners 0.08: 120 / 104 / -      122 / 107 / -
+//   candidates 1.5, partners 0.15: 82 / 73 / 86       85 / 72 / 88
+//   candidates 3.8, partners 0.38: 64 / 58 / 60       65 / 59 / 62
+//   candidates 5.3, partners 0.53: - / 59 / 58        - / 61 / 63
+//   candidates 7.6, partners 0.76: - / 68 / 57        - / 68 / 62
+//   candidates 22, partners 2.3:   74 / - / 63        81 / - / 77
+// and 1M particles in four species (6, 0.32) 95 / 100 / 98, 256 replicas (3.8,
+// 0.4) 205 / 187 / 204, the 16 crowded cytosol boxes (49, 2.1) 179 / - / 159,
+// after 600 steps 485 / - / 402.  The pieces of a composite (`ext`) gather the
+// particles, so that the mean says little and many a wave lists in vain: the 2M
+// slab without one 205 / 184 / -, with one after 200 steps 556 / 562 / 545.
+static int force_form(const RdDev& P, const std::vector<RdRep>& reps, bool ext)
 {
-    if (P.S != 1 || !P.n_pot2) return false;    // the walk is of the nearest cells
-    double n = 0.0, vol = 0.0, rc3 = 0.0;
+    if (P.S != 1 || !P.n_pot2) return RD_FORM_ROWS;     // both walk the nearest cells
+    double n = 0.0, cells = 0.0, vol = 0.0, rc3 = 0.0;
     for (const RdRep& R : reps) {
-        if (R.L[0] < 3 || R.L[1] < 3 || R.L[2] < 3) return false;   // a cell may not be met twice
+        if (R.L[0] < 3 || R.L[1] < 3 || R.L[2] < 3) return RD_FORM_ROWS;    // a cell may not be met twice
         n += R.n;
+        cells += (double)R.L[0] * R.L[1] * R.L[2];
         vol += (double)R.Lb[0] * R.Lb[1] * R.Lb[2];
     }
-    for (int k = 0; k < P.nt * P.nt; ++k) rc3 += std::pow((double)P.rc2[k], 1.5);
-    return n * (4.0 / 3.0 * M_PI) * rc3 / ((double)P.nt * P.nt) >= 0.35 * vol;
+    for (int k = 0; k < P.nt; ++k)
+        for (int l = 0; l < P.nt; ++l) rc3 += std::pow((double)P.rc2[k * P.nt + l], 1.5);
+    if (!ext && 27.0 * n <= 5.0 * cells) return RD_FORM_SPARSE;
+    return n * (4.0 / 3.0 * M_PI) * rc3 / ((double)P.nt * P.nt) >= 0.35 * vol ? RD_FORM_DEALT : RD_FORM_ROWS;
 }
 
 double rd_host_r0(const rd_system* h, int i, int j)
@@ -1343,7 +1360,7 @@ static int build_tables(rd_system* h)
             wave_tab.push_back(w);
         }
     }
-    h->queue_form = queue_form_pays(P, rep_dev);
+    for (int ext = 0; ext < 2; ++ext) h->force_form[ext] = force_form(P, rep_dev, ext);
     h->P = P;
     h->max_range = maxr;
     h->max_rxn = maxrx;
@@ -1650,18 +1667,20 @@ static void launch_force_ppt(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 void rd_host_launch_force(rd_system* h, hipEvent_t ev0, hipEvent_t ev1)
 {
     if (h->n <= 0) return;
-    if (h->kern == RD_KERNEL_GATHER && h->block == 256 && h->ppt == 1 && lanes_per_particle(h) == 1 && h->queue_form) {
+    const int form = h->force_form[h->ext_active()];
+    if (h->kern == RD_KERNEL_GATHER && h->block == RD_BLOCK && h->ppt == 1 && lanes_per_particle(h) == 1 && form != RD_FORM_ROWS) {
         const dim3 grid(wave_blocks(h));
+        auto* const kernel = form == RD_FORM_SPARSE ? k_force_update_sparse : k_force_update_dealt;
         if (ev0)
-            hipExtLaunchKernelGGL(k_force_update_dealt, grid, dim3(RD_BLOCK), 0, h->stream, ev0, ev1, 0,
+            hipExtLaunchKernelGGL(kernel, grid, dim3(RD_BLOCK), 0, h->stream, ev0, ev1, 0,
                                   (const float4*)h->d_ps, h->d_pn, h->d_kr, h->d_count, h->d_bsum,
                                   (const uint32_t*)h->d_start, (const RdDev*)h->d_P, (const RdRep*)h->d_reps,
                                   (const RdWave*)h->d_waves, h->nwaves, (const RdPot1Dev*)h->d_pot1, h->d_st,
                                   (const float*)h->d_noise, h->n);
         else
-            hipLaunchKernelGGL(k_force_update_dealt, grid, dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_pn, h->d_kr,
-                               h->d_count, h->d_bsum, h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1,
-                               h->d_st, h->d_noise, h->n);
+            hipLaunchKernelGGL(kernel, grid, dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_pn, h->d_kr, h->d_count,
+                               h->d_bsum, h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_st,
+                               h->d_noise, h->n);
         return;
     }
     switch (lanes_per_particle(h)) {

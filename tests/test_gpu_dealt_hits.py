@@ -51,8 +51,8 @@ def boxes(cells, nmin, nmax, clump=1.0, seed=5):
     ((4, 3, 5), 60, 66, 1.0),
     ((7, 4, 3), 1, 200, 0.5),
     ((2, 3, 3), 20, 70, 1.0),           # two cells per axis: not the queue's
-    ((8, 8, 8), 80, 80, 1.0),           # 0.43 partners
-    ((8, 8, 8), 50, 50, 1.0),           # 0.27 partners: below the rule
+    ((8, 8, 8), 110, 110, 1.0),         # 5.8 candidates, 0.6 partners
+    ((8, 8, 8), 80, 80, 1.0),           # 4.2 candidates: the sparse form's
 ], ids=str)
 def test_boxes(cells, nmin, nmax, clump):
     spec, bounds, counts, xyz, types = boxes(cells, nmin, nmax, clump)
