@@ -165,6 +165,7 @@ struct rd_system {
     uint32_t comp_mask = 0;
     bool comp_sum = false;           // RD_COMBINE_SUM: sum of the pieces (else nearest piece)
     int npieces = 0;
+    bool comp_allz = false;          // every piece's axis is +z
     void* d_pieces = nullptr;
     uint16_t* d_comp_list = nullptr; // candidate lists of the nearest-piece grid (comp_cells cells)
     long comp_cells = 0;

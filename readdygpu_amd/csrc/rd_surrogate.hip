@@ -95,6 +95,32 @@ __device__ __forceinline__ float4 composite_at(const RdPiece* __restrict__ pc, i
     return make_float4(g.x, g.y, g.z, best);
 }
 
+// The nearest of pieces whose axes are all +z, the same arithmetic as
+// piece_energy: a[k] = origin, radius; b[k] = half height, k / 2 (in LDS).
+// Bound by vector instructions: a piece is two LDS reads, of which four
+// pieces' go out together, and 16 instructions and a square root, where the
+// form for any axis reads ten words and branches on each piece's axis.  256
+// disks, 16 crowded cytosol boxes: pass 90 -> 68 us, whole step 264 -> 240; 64
+// boxes 806 -> 764.  The pieces from scalar loads: 272 (16 boxes).
+__device__ __forceinline__ float4 composite_at_z(const float4* __restrict__ a, const float2* __restrict__ b,
+                                                 const RdPiece* __restrict__ pieces, int np, float x, float y, float z)
+{
+    float best = INFINITY;
+    int kb = 0;
+#pragma unroll 4
+    for (int k = 0; k < np; ++k) {
+        const float4 o = a[k];
+        const float2 h = b[k];
+        const float vx = x - o.x, vy = y - o.y, vz = z - o.z;
+        const float dn = fmaxf(fabsf(vz) - h.x, 0.0f);
+        const float dr = fmaxf(__builtin_amdgcn_sqrtf(vx * vx + vy * vy) - o.w, 0.0f);
+        const float e = h.y * (dn * dn + dr * dr);
+        if (e < best) { best = e; kb = k; }
+    }
+    const float3 g = piece_grad(pieces[kb], x, y, z);
+    return make_float4(g.x, g.y, g.z, best);
+}
+
 // ---- nearest piece by a grid of candidate lists ----
 // The domain (the union of the replica boxes) is cut into cells; each cell
 // lists, in index order, the pieces that can be the nearest in energy
@@ -250,20 +276,32 @@ __global__ __launch_bounds__(256) void k_composite_points_near(const float* __re
 // contiguous shares would be unbalanced), and compacts the selected ones
 // into an LDS queue; whenever 256 are queued, every thread evaluates one, so
 // no lane idles on an unselected particle.
-// Piece table in dynamic LDS: np * sizeof(RdPiece) bytes.
-template <bool SUM>
+// Piece table in dynamic LDS: np * sizeof(RdPiece) bytes; ALLZ: every piece's
+// axis is +z.
+template <bool SUM, bool ALLZ>
 __global__ __launch_bounds__(256) void k_composite_slots(const float4* __restrict__ ps, int n,
                                                          const RdPiece* __restrict__ pieces, int np,
                                                          uint32_t type_mask, float4* __restrict__ gext)
 {
-    extern __shared__ RdPiece pc[];
+    extern __shared__ __align__(16) RdPiece pc[];
     __shared__ uint32_t q[512];
     __shared__ int wcnt[4];
-    for (int k = threadIdx.x; k < np; k += 256) pc[k] = pieces[k];
+    float4* const za = reinterpret_cast<float4*>(pc);
+    float2* const zb = reinterpret_cast<float2*>(za + np);
+    for (int k = threadIdx.x; k < np; k += 256) {
+        if constexpr (ALLZ) {
+            const RdPiece p = pieces[k];
+            za[k] = make_float4(p.o[0], p.o[1], p.o[2], p.R);
+            zb[k] = make_float2(p.hh, 0.5f * p.k);
+        } else {
+            pc[k] = pieces[k];
+        }
+    }
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     auto eval = [&](uint32_t s) {
         float4 p = ps[s];
-        gext[s] = composite_at<SUM>(pc, np, p.x, p.y, p.z);
+        if constexpr (ALLZ) gext[s] = composite_at_z(za, zb, pieces, np, p.x, p.y, p.z);
+        else gext[s] = composite_at<SUM>(pc, np, p.x, p.y, p.z);
     };
     int qn = 0;                       // queued entries (same in every thread)
     for (long base = (long)xcd_block(blockIdx.x, gridDim.x) * 256; base < n; base += (long)gridDim.x * 256) {
@@ -1139,6 +1177,13 @@ static int comp_grid(rd_system* h, RdCompGrid* g)
 // persistent grid of k_mlp_points: one tile of 16 points per wave and round
 static inline unsigned mlp_point_blocks(long m) { return (unsigned)std::min(((m + 15) / 16 + 3) / 4, 2048L); }
 
+// the exact pass over the slots of some types
+static auto* slots_kernel(const rd_system* h)
+{
+    return h->comp_sum ? k_composite_slots<true, false>
+                       : (h->comp_allz ? k_composite_slots<false, true> : k_composite_slots<false, false>);
+}
+
 // external pass of the step (sorted slots -> gext)
 void rd_host_launch_ext(rd_system* h)
 {
@@ -1150,7 +1195,7 @@ void rd_host_launch_ext(rd_system* h)
     } else if ((h->comp_mask & all_types(h)) == all_types(h)) {
         // (a composite on some of the types keeps the scan below: it is the
         // reference that the surrogate is trained for and timed against on
-        // the cytosol's membrane, 64 replicas: scan 217 us, surrogate 101 us,
+        // the cytosol's membrane, 64 replicas: scan 200 us, surrogate 91 us,
         // grid 64 us)
         if (h->comp_near.list)
             hipLaunchKernelGGL(k_composite_near, dim3(nb256(h->n)), dim3(256), 0, h->stream, h->d_ps, h->n,
@@ -1161,8 +1206,7 @@ void rd_host_launch_ext(rd_system* h)
                            h->d_gext);
     } else {
         unsigned blocks = std::min(h->ext_blocks[0] > 0 ? (unsigned)h->ext_blocks[0] : 2048u, nb256(h->n));
-        hipLaunchKernelGGL(h->comp_sum ? k_composite_slots<true> : k_composite_slots<false>, dim3(blocks), dim3(256),
-                           pieces_lds(h), h->stream, h->d_ps, h->n, (const RdPiece*)h->d_pieces, h->npieces,
+        hipLaunchKernelGGL(slots_kernel(h), dim3(blocks), dim3(256), pieces_lds(h), h->stream, h->d_ps, h->n, (const RdPiece*)h->d_pieces, h->npieces,
                            h->comp_mask, h->d_gext);
     }
 }
@@ -1178,7 +1222,7 @@ int rd_host_ext_capacity(rd_system* h)
         if (rc) return rc;
     }
     int per = 0;
-    SHIPCK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_composite_slots<false>, 256,
+    SHIPCK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)slots_kernel(h), 256,
                                                            pieces_lds(h)));
     h->ext_blocks[0] = std::max(per, 1) * h->ncu;
     SHIPCK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_mlp_slots, 256, 0));
@@ -1215,8 +1259,8 @@ extern "C" int rd_set_composite(rd_system* h, int n_pieces, const rd_pot1* piece
     static bool attr = false;
     if (!attr) {
         const int bytes = (int)(sizeof(RdPiece) * RD_PIECES_MAX);
-        const void* fns[] = { (const void*)k_composite_slots<false>, (const void*)k_composite_slots<true>,
-                              (const void*)k_composite_all<false>, (const void*)k_composite_all<true>,
+        const void* fns[] = { (const void*)k_composite_slots<false, false>, (const void*)k_composite_slots<false, true>,
+                              (const void*)k_composite_slots<true, false>, (const void*)k_composite_all<false>, (const void*)k_composite_all<true>,
                               (const void*)k_composite_points<false>, (const void*)k_composite_points<true>,
                               (const void*)k_sur_data<false, false>, (const void*)k_sur_data<true, false>,
                               (const void*)k_comp_grid };
@@ -1238,6 +1282,7 @@ extern "C" int rd_set_composite(rd_system* h, int n_pieces, const rd_pot1* piece
         SHIPCK(h, hipMemcpy(h->d_pieces, pc.data(), sizeof(RdPiece) * n_pieces, hipMemcpyHostToDevice));
     }
     h->comp_grid_set = false;
+    h->comp_allz = std::all_of(pc.begin(), pc.end(), [](const RdPiece& p) { return p.zaxis != 0; });
     h->npieces = n_pieces;
     h->comp_mask = type_mask;
     h->comp.assign(pieces, pieces + n_pieces);
