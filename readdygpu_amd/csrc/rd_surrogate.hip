@@ -1195,7 +1195,7 @@ void rd_host_launch_ext(rd_system* h)
     } else if ((h->comp_mask & all_types(h)) == all_types(h)) {
         // (a composite on some of the types keeps the scan below: it is the
         // reference that the surrogate is trained for and timed against on
-        // the cytosol's membrane, 64 replicas: scan 200 us, surrogate 91 us,
+        // the cytosol's membrane, 64 replicas: scan 189 us, surrogate 91 us,
         // grid 64 us)
         if (h->comp_near.list)
             hipLaunchKernelGGL(k_composite_near, dim3(nb256(h->n)), dim3(256), 0, h->stream, h->d_ps, h->n,
