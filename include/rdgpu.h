@@ -365,7 +365,9 @@ typedef struct {
                               testing distances first and evaluating the listed hits after, one
                               workgroup per group of 64-slot work items; at 256 threads and one particle
                               per lane, systems too small to fill the chip (up to 8 work items per
-                              compute unit) take 3 or 9 lanes per particle.  QUEUE: the same per-lane
+                              compute unit) take 3 or 9 lanes per particle, sparse ones list a
+                              particle's candidates before testing them and crowded ones deal a
+                              wave's hits to its lanes.  QUEUE: the same per-lane
                               work on a resident grid (occupancy x compute units) whose workgroups
                               each own a contiguous share of the work items, taken by their waves
                               from a ticket in LDS until none are left (ppt is ignored).
