@@ -133,9 +133,12 @@ __device__ __forceinline__ float4 composite_at_z(const float4* __restrict__ a, c
 // k/2 (d(centre) + rho)^2 over all pieces cannot be nearest.  Of the pieces
 // left, those after a piece that contains the whole cell (energy 0) never
 // come first.  Coplanar pieces (z axis, same plane, height and stiffness)
-// share their axial term, so among those of the nearest piece's plane only
-// the radial excess max(r - R, 0) decides: one that exceeds another's
-// everywhere in the cell is left out, and so is one after a coplanar piece
+// share their axial term dn, so among those of the nearest piece's plane only
+// the radial excess dr = max(r - R, 0) decides: one whose excess is larger
+// than another's everywhere in the cell is left out, if the scan's FP32 sum
+// dn^2 + dr^2 tells them apart, that is if the squared excesses differ by more
+// than its rounding (far from the plane the sum absorbs dr, both energies are
+// the same and the lower index wins); and so is one after a coplanar piece
 // that covers the cell's whole x-y extent (a membrane of overlapping disks).
 #define RD_GRID_CELLS (1 << 16)
 #define RD_GRID_LIST 32          // entry 0: count (0xffff: scan all pieces), then indices
@@ -186,13 +189,16 @@ __global__ __launch_bounds__(256) void k_comp_grid(RdCompGrid g, float margin, c
         (void)dist(pieces[k], &r);
         if (coplanar(ref, pieces[k])) side = fminf(side, fmaxf(r - pieces[k].R, 0.0f) + rhoxy);
     }
+    const float axial = fmaxf(fabsf(z - ref.o[2]) - ref.hh, 0.0f) + rho;     // their dn, at most
     uint16_t* out = list + (size_t)c * RD_GRID_LIST;
     int cnt = 0, cover = -1;
     for (int k = 0; k < np; ++k) {
         const RdPiece& p = pieces[k];
         const float d = fmaxf(dist(p, &r) - rho, 0.0f);
         if (!(0.5f * p.k * d * d <= least)) continue;
-        if (coplanar(ref, p) && r - p.R - rhoxy > side) continue;
+        // (3.6e-7 of the sum: the roundings of both sums and of their products with k / 2)
+        const float a = r - p.R - rhoxy;
+        if (coplanar(ref, p) && a > side && (a - side) * (a + side) > 1e-6f * (axial * axial + a * a)) continue;
         if (cover >= 0 && coplanar(p, pieces[cover])) continue;
         if (++cnt >= RD_GRID_LIST) break;
         out[cnt] = (uint16_t)k;
