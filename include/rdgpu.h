@@ -140,7 +140,10 @@ int rd_set_particles(rd_system* h, int n, const float* xyz, const int* type);
  * Reactions need a single-system handle. */
 int rd_set_replicas(rd_system* h, int n_replicas, const double* bounds, const uint32_t* streams,
                     const int* counts, const float* xyz, const int* type);
-/* CudaSimulation::initialize: upload tables, build the first cell list */
+/* CudaSimulation::initialize: upload tables, build the first cell list.  A
+ * second call uploads again the positions and types that were last set or
+ * copied out (rd_copy_pos_from_device), as the reference its host arrays, or
+ * those that rd_apply_reactions left; the step counter goes on. */
 int rd_initialize(rd_system* h);
 
 /* ---- the step: Simulation::simulate(int) (Simulation.cpp:349-355) ->

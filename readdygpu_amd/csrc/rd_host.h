@@ -14,6 +14,9 @@
 
 struct RdStepState;
 
+// where the positions and types last set or copied out are (rd_system::mirror)
+enum { RD_MIRROR_HOST, RD_MIRROR_DEVICE, RD_MIRROR_NONE };
+
 // forms of the force kernel's gather (force_form in rd_system.hip)
 enum { RD_FORM_ROWS, RD_FORM_SPARSE, RD_FORM_DEALT };
 
@@ -51,10 +54,14 @@ struct rd_system {
     int force_form[2] = {};          // the step's force kernel at one particle per lane, without
                                      // and with an external pass (RD_FORM_*)
 
-    // particles in index order (host mirror)
+    // particles in index order: as last set or copied out, which is what
+    // rd_initialize uploads.  After a copy into a caller's arrays they are in
+    // d_xyz_io (RD_MIRROR_DEVICE: 3n coordinates, n types) and the host arrays
+    // are behind; after reactions (RD_MIRROR_NONE) only the sorted state is.
     int n = 0;
     std::vector<float> hxyz;
     std::vector<int> htype;
+    int mirror = RD_MIRROR_HOST;
 
     bool initialized = false;
     bool dirty = true;            // tables changed

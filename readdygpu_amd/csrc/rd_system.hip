@@ -1405,6 +1405,7 @@ extern "C" int rd_set_particles(rd_system* h, int n, const float* xyz, const int
     h->n = n;
     h->hxyz.assign(xyz, xyz + 3 * (size_t)n);
     h->htype.assign(type, type + n);
+    h->mirror = RD_MIRROR_HOST;
     h->tcount.assign((size_t)h->nt, 0);
     for (int i = 0; i < n; ++i) h->tcount[type[i]]++;
     h->snap_valid = false;
@@ -1444,6 +1445,7 @@ extern "C" int rd_set_replicas(rd_system* h, int nrep, const double* bounds, con
     h->n = (int)total;
     h->hxyz.assign(xyz, xyz + 3 * (size_t)total);
     h->htype.assign(type, type + total);
+    h->mirror = RD_MIRROR_HOST;
     h->tcount.assign((size_t)nrep * h->nt, 0);
     base = 0;
     for (int r = 0; r < nrep; ++r)
@@ -1546,11 +1548,11 @@ static void launch_sort(rd_system* h, int advance)
                        (const uint32_t*)h->d_gid, h->d_slot, h->d_bsum, h->nscan);
 }
 
-// particles of the io arrays into slot form, cell histogram and tile sums
-static void launch_pack(rd_system* h)
+// particles in index order into slot form, cell histogram and tile sums
+static void launch_pack(rd_system* h, const float* xyz, const int* type)
 {
-    hipLaunchKernelGGL(k_pack, dim3(nblk(h->n, RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream, h->d_xyz_io, h->d_type_io,
-                       h->d_rep_of, h->n, h->d_reps, h->d_pn, h->d_kr, h->d_count, h->d_gid);
+    hipLaunchKernelGGL(k_pack, dim3(nblk(h->n, RD_BLOCK)), dim3(RD_BLOCK), 0, h->stream, xyz, type, h->d_rep_of, h->n,
+                       h->d_reps, h->d_pn, h->d_kr, h->d_count, h->d_gid);
     hipLaunchKernelGGL(k_scan_reduce, dim3(h->nscan), dim3(RD_BLOCK), 0, h->stream, h->d_count, h->ncell, h->d_bsum);
 }
 
@@ -1821,7 +1823,7 @@ static int upload(rd_system* h)
             HIPCK(h, hipMemcpyAsync(h->d_type_io, h->htype.data(), sizeof(int) * h->n, hipMemcpyHostToDevice,
                                     h->stream));
         }
-        launch_pack(h);
+        launch_pack(h, h->d_xyz_io, h->d_type_io);
     }
     launch_sort(h, 0);
     HIPCK(h, hipGetLastError());
@@ -1842,6 +1844,17 @@ extern "C" int rd_initialize(rd_system* h)
     HIPCK(h, hipSetDevice(h->dev));
     int rc = scratch_setup(h);
     if (rc) return rc;
+    // a second call: the host arrays may be behind
+    if (h->mirror == RD_MIRROR_NONE) {
+        rc = rd_copy_pos_from_device(h, nullptr, nullptr);
+        if (rc) return rc;
+    } else if (h->mirror == RD_MIRROR_DEVICE) {
+        const size_t n = (size_t)h->n;
+        HIPCK(h, hipMemcpyAsync(h->hxyz.data(), h->d_xyz_io, 12 * n, hipMemcpyDeviceToHost, h->stream));
+        HIPCK(h, hipMemcpyAsync(h->htype.data(), h->d_xyz_io + 3 * n, 4 * n, hipMemcpyDeviceToHost, h->stream));
+        HIPCK(h, hipStreamSynchronize(h->stream));
+        h->mirror = RD_MIRROR_HOST;
+    }
     rc = upload(h);
     if (rc) return rc;
     h->initialized = true;
@@ -1943,6 +1956,7 @@ int rd_host_set_state(rd_system* h, const std::vector<float>& xyz, const std::ve
     if (xyz.size() != 3 * (size_t)h->n || type.size() != (size_t)h->n) return set_err(h, RD_EINVAL, "state size");
     h->hxyz = xyz;
     h->htype = type;
+    h->mirror = RD_MIRROR_HOST;
     h->particles_dirty = true;
     return RD_OK;
 }
@@ -1983,12 +1997,14 @@ extern "C" int rd_copy_pos_from_device(rd_system* h, float* xyz, int* type)
     const size_t n = (size_t)h->n;
     if (n > 0) {
         // types behind the positions, so that one copy brings both; without a
-        // destination the host mirrors are refreshed
+        // destination they go to the host arrays of the handle
         int* dtype = (int*)(h->d_xyz_io + 3 * n);
         hipLaunchKernelGGL(k_unsort, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_reps,
                            h->d_waves, h->nwaves, h->d_xyz_io, dtype);
         HIPCK(h, hipGetLastError());
-        if (!xyz && !type) { xyz = h->hxyz.data(); type = h->htype.data(); }
+        h->mirror = RD_MIRROR_NONE;
+        const bool own = !xyz && !type;
+        if (own) { xyz = h->hxyz.data(); type = h->htype.data(); }
         char* stage = rd_host_stage(h, 16 * n);
         if (stage) {
             HIPCK(h, hipMemcpyAsync(stage, h->d_xyz_io, 16 * n, hipMemcpyDeviceToHost, h->stream));
@@ -1999,6 +2015,7 @@ extern "C" int rd_copy_pos_from_device(rd_system* h, float* xyz, int* type)
         HIPCK(h, hipStreamSynchronize(h->stream));
         if (stage && xyz) memcpy(xyz, stage, 12 * n);
         if (stage && type) memcpy(type, stage + 12 * n, 4 * n);
+        h->mirror = own ? RD_MIRROR_HOST : RD_MIRROR_DEVICE;
         return RD_OK;
     }
     HIPCK(h, hipStreamSynchronize(h->stream));
@@ -2026,21 +2043,23 @@ extern "C" int rd_gradients(rd_system* h, float* grad, double* energy)
     if (rc) return rc;
     if (h->n == 0) { if (energy) *energy = 0.0; return RD_OK; }
     double* const d_etot = (double*)((char*)h->d_st + offsetof(RdStepState, etot));
+    // (the next step's records are not in use between steps; the io array may
+    // hold the particles as last copied out)
+    float* const d_grad = (float*)h->d_pn;
     HIPCK(h, hipMemsetAsync(d_etot, 0, sizeof(double), h->stream));
     if (h->ext_active()) rd_host_launch_ext(h);
     if (h->nwaves <= 3 * h->ncu)     // the line of lanes_per_particle
         hipLaunchKernelGGL((k_gradients_spread<9>), dim3(std::max(1, h->nwaves)), dim3(64 * 9), 0, h->stream, h->d_ps,
-                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, d_etot,
-                           h->d_st);
+                           h->d_start, h->d_P, h->d_reps, h->d_waves, h->nwaves, h->d_pot1, d_grad, d_etot, h->d_st);
     else
         hipLaunchKernelGGL(k_gradients, dim3(wave_blocks(h)), dim3(RD_BLOCK), 0, h->stream, h->d_ps, h->d_start, h->d_P,
-                           h->d_reps, h->d_waves, h->nwaves, h->d_pot1, h->d_xyz_io, d_etot, h->d_st);
+                           h->d_reps, h->d_waves, h->nwaves, h->d_pot1, d_grad, d_etot, h->d_st);
     HIPCK(h, hipGetLastError());
     const size_t bytes = grad ? sizeof(float) * 3 * (size_t)h->n : 0;
     RdStepState st;
     char* stage = rd_host_stage(h, sizeof(st) + bytes);
     if (bytes)
-        HIPCK(h, hipMemcpyAsync(stage ? (void*)(stage + sizeof(st)) : (void*)grad, h->d_xyz_io, bytes,
+        HIPCK(h, hipMemcpyAsync(stage ? (void*)(stage + sizeof(st)) : (void*)grad, d_grad, bytes,
                                 hipMemcpyDeviceToHost, h->stream));
     rc = read_state(h, &st);
     if (rc) return rc;
@@ -2497,6 +2516,7 @@ static int apply_reactions(rd_system* h, const float* cr, const int* creation_re
     }
     const int n_new = noff[R];
     if (n_new > RD_MAX_PARTICLES) return set_err(h, RD_EINVAL, "too many particles");
+    h->mirror = RD_MIRROR_NONE;      // the io arrays are written anew
     if (n_new > h->cap) {
         rc = grow_particles(h, n_new, true);
         if (rc) return rc;
@@ -2554,7 +2574,7 @@ static int apply_reactions(rd_system* h, const float* cr, const int* creation_re
     if (e != hipSuccess || se != hipSuccess)
         return set_err(h, RD_EHIP, std::string("reaction compaction: ") + hipGetErrorString(e != hipSuccess ? e : se));
     memcpy(delcnt.data(), lists, sizeof(uint32_t) * delcnt.size());
-    // particle counts per (replica, type); the host position/type mirrors are
+    // particle counts per (replica, type); the host arrays of the handle are
     // refreshed from the device when next read
     for (size_t k = 0; k < delcnt.size(); ++k) h->tcount[k] -= (long)delcnt[k];
     for (const Born& b : born) h->tcount[(size_t)b.rep * nt + b.type]++;
@@ -2669,18 +2689,12 @@ extern "C" int rd_frame_rewind(rd_system* h)
     if (!h) return RD_EINVAL;
     if (!h->snap_valid || h->snap_n != h->n) return set_err(h, RD_ESTATE, "no frame copy of the current particle set");
     HIPCK(h, hipStreamSynchronize(h->stream));
-    if (h->n > 0) {
-        HIPCK(h, hipMemcpyAsync(h->d_xyz_io, h->d_snap_xyz, sizeof(float) * 3 * (size_t)h->n,
-                                hipMemcpyDeviceToDevice, h->stream));
-        HIPCK(h, hipMemcpyAsync(h->d_type_io, h->d_snap_type, sizeof(int) * (size_t)h->n, hipMemcpyDeviceToDevice,
-                                h->stream));
-    }
     int rc = rd_host_set_step(h, h->snap_step);
     if (rc) return rc;
     // same particle set and tables: pack the snapshot and sort it again (the
     // captured step graphs stay valid)
     if (h->n > 0)
-        launch_pack(h);
+        launch_pack(h, h->d_snap_xyz, h->d_snap_type);
     launch_sort(h, 0);
     HIPCK(h, hipGetLastError());
     HIPCK(h, hipStreamSynchronize(h->stream));
