@@ -1051,6 +1051,16 @@ static void free_frames(rd_system* h)
     h->snap_cap = 0; h->snap_valid = false;
 }
 
+// tables as last uploaded: none (a table there is taken for one whose copy, and
+// whatever follows from it on the device, was enqueued)
+static void forget_uploads(rd_system* h)
+{
+    h->P_up_set = false;
+    h->reps_up.clear();
+    h->waves_up.clear();
+    h->pot1_up.clear();
+}
+
 static void free_dev(rd_system* h)
 {
     free_bonds(h);
@@ -1069,7 +1079,7 @@ static void free_dev(rd_system* h)
     h->d_poff = nullptr; h->d_pbs = nullptr; h->d_pkeep = nullptr; h->poff_cap = 0;
     h->d_xyz_io = nullptr; h->d_type_io = nullptr; h->d_react = nullptr; h->react_cap = 0;
     stage_release(h);
-    h->P_up_set = false; h->reps_up.clear(); h->waves_up.clear(); h->pot1_up.clear();
+    forget_uploads(h);
     h->d_reps = nullptr; h->d_waves = nullptr; h->d_rep_of = nullptr;
     h->cap = 0; h->ncell_alloc = 0; h->pairs_cap = 0; h->noise_cap = 0; h->nrep_alloc = 0; h->nwave_alloc = 0;
 }
@@ -1756,8 +1766,7 @@ static int upload_bonds(rd_system* h)
     return RD_OK;
 }
 
-// upload tables and particles, build the cell-sorted arrays
-static int upload(rd_system* h)
+static int upload_all(rd_system* h)
 {
     int rc = build_tables(h);
     if (rc) return rc;
@@ -1832,6 +1841,14 @@ static int upload(rd_system* h)
     h->particles_dirty = false;
     drop_graph(h);
     return RD_OK;
+}
+
+// upload tables and particles, build the cell-sorted arrays
+static int upload(rd_system* h)
+{
+    const int rc = upload_all(h);
+    if (rc) forget_uploads(h);      // the next call brings up everything again
+    return rc;
 }
 
 static int scratch_setup(rd_system* h);
