@@ -29,6 +29,7 @@ extern "C" int rd_bench_steps(rd_system* h, int nsteps, double* out)
 {
     if (!h || nsteps < 1 || !out) return RD_EINVAL;
     int rc = rd_host_refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, RD_GRID_NOW);
     if (rc) return rc;
     std::vector<hipEvent_t> ev(5 * (size_t)nsteps, nullptr);
     hipGraph_t g = nullptr;
@@ -122,6 +123,7 @@ extern "C" int rd_bench_ext(rd_system* h, int reps, double* avg_ms)
 {
     if (!h || reps < 1 || !avg_ms) return RD_EINVAL;
     int rc = rd_host_refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, RD_GRID_NOW);
     if (rc) return rc;
     if (!h->ext_active()) {
         h->err = "no external pass (set a composite first)";
@@ -148,6 +150,7 @@ extern "C" int rd_bench_steps_direct(rd_system* h, int nsteps, double* out)
 {
     if (!h || nsteps < 1 || !out) return RD_EINVAL;
     int rc = rd_host_refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, RD_GRID_NOW);
     if (rc) return rc;
     std::vector<hipEvent_t> ev(5 * (size_t)nsteps, nullptr);
     double tf = 0.0, ts = 0.0, te = 0.0;

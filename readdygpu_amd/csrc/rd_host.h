@@ -176,7 +176,9 @@ struct rd_system {
     void* d_pieces = nullptr;
     uint16_t* d_comp_list = nullptr; // candidate lists of the nearest-piece grid (comp_cells cells)
     long comp_cells = 0;
-    bool comp_grid_set = false;      // built for the pieces and this domain
+    bool comp_grid_set = false;      // comp_built is of the pieces and this domain
+    RdCompGrid comp_built{};
+    long comp_passes = 0;            // passes over them since (comp_grid)
     double comp_lo[3] = { 0, 0, 0 }, comp_hi[3] = { 0, 0, 0 };
     RdCompGrid comp_near{};          // of the step's external pass
     int ext_mode = RD_EXT_EXACT;
@@ -212,4 +214,7 @@ void rd_host_launch_force(rd_system* h, hipEvent_t ev0 = nullptr, hipEvent_t ev1
 void rd_host_launch_sort(rd_system* h, int advance);
 void rd_host_launch_ext(rd_system* h);
 int rd_host_ext_capacity(rd_system* h);
+#define RD_GRID_NOW (1L << 20)
+int rd_host_ext_passes(rd_system* h, long passes, bool* changed);
+int rd_host_passes(rd_system* h, long passes);
 void rd_host_free_surrogate(rd_system* h);

@@ -236,8 +236,9 @@ __device__ __forceinline__ float4 composite_near(const RdCompGrid& g, const RdPi
         const float e = piece_energy(p, x, y, z);
         if (e < best) { best = e; kb = k; }
     };
-    uint4 v = l[0];                              // the count and the first seven entries
-    const int cnt = in ? (int)(v.x & 0xffffu) : 0xffff;
+    uint4 v = make_uint4(0xffffu, 0u, 0u, 0u);
+    if (in) v = l[0];                            // the count and the first seven entries
+    const int cnt = (int)(v.x & 0xffffu);
     if (!__any(act && cnt == 0xffff)) {
         for (int i = 1; act && i <= cnt;) {
             const uint32_t w[4] = { v.x, v.y, v.z, v.w };
@@ -278,8 +279,8 @@ __device__ __forceinline__ float4 composite_near(const RdCompGrid& g, const RdPi
 // type.  Bound by the lists' and pieces' load latency.  512 pieces, 500,000
 // particles of the slab: 16 us (9.4 us after 100 steps, when they lie near the
 // pieces) against 147 us (129) scanning all pieces from LDS; 2M: 43 against
-// 503 us; 16 pieces: 8.0 against 7.9 us (4.9 against 7.5), so the grid is used
-// from 9 pieces on.  Twice the cells: 14 us, for twice the set-up.
+// 503 us; 16 pieces: 5.8 against 7.8 us.  Twice the cells: 14 us, for twice the
+// set-up.  When it is built and used: comp_grid.
 __global__ __launch_bounds__(256) void k_composite_near(const float4* __restrict__ ps, int n, RdCompGrid g,
                                                         const RdPiece* __restrict__ pieces, int np,
                                                         float4* __restrict__ gext)
@@ -1164,59 +1165,93 @@ void rd_host_free_surrogate(rd_system* h)
 
 static uint32_t all_types(const rd_system* h) { return h->nt >= 32 ? 0xffffffffu : (1u << h->nt) - 1u; }
 
-// Grid of the nearest-piece composite over the union of the replica boxes,
-// built when the pieces or the boxes have changed (k_comp_grid on the handle's
-// stream).  Not used, and every piece scanned, for few pieces, a sum, or a
-// stiffness that is not positive (no nearest distance).
-#define RD_GRID_MIN_PIECES 8
-static int comp_grid(rd_system* h, RdCompGrid* g)
+// Grid of the nearest-piece composite over the union of the replica boxes, for
+// a call that passes over the pieces `passes` times (of passes_of; 0: only a
+// grid that is there is taken, RD_GRID_NOW: the caller asks for it).
+// Not used, and every piece scanned, for a sum, a stiffness that is not positive
+// (no nearest distance) or few pieces: on sorted slots 12 pieces win and 9 do
+// not (2M slots: scan 18.5 and 16.2 us, grid 16.6 and 17.1), on points in random
+// order, whose lists are read here and there, 32 and 24 (1M training points:
+// scan 58.0 and 54.5 us, grid 57.5 and 56.9).
+// Building the lists (k_comp_grid on the handle's stream) takes as long as 3.5
+// passes save, at any number of pieces (512: 200 us for 55 us a pass; 2,048:
+// 780 for 220), so it waits until more than three passes over the same pieces
+// and boxes have been asked for: a program that moves its pieces for every few
+// points or steps scans them (512 pieces, one point: 474 us for rd_set_composite
+// and rd_composite_eval, 667 with a grid).
+#define RD_GRID_SLOT_PIECES 12
+#define RD_GRID_POINT_PIECES 32
+#define RD_GRID_PASSES 3
+// A scan takes the same time for up to about 130,000 points, which are resident
+// at once, and grows from there.
+static long passes_of(long points) { return 1 + (points >> 17); }
+
+// union of the replica boxes: [axis] { low, high }
+static void union_box(const rd_system* h, double (&box)[3][2])
+{
+    for (int d = 0; d < 3; ++d) {
+        box[d][0] = h->reps.empty() ? h->prm.lattice_bounds[2 * d] : h->reps[0].lo[d];
+        box[d][1] = h->reps.empty() ? h->prm.lattice_bounds[2 * d + 1] : h->reps[0].hi[d];
+        for (const rd_system::Rep& r : h->reps) {
+            box[d][0] = std::min(box[d][0], r.lo[d]);
+            box[d][1] = std::max(box[d][1], r.hi[d]);
+        }
+    }
+}
+
+static int comp_grid(rd_system* h, RdCompGrid* g, long passes, int min_pieces)
 {
     memset(g, 0, sizeof(*g));
-    if (h->comp_sum || h->npieces <= RD_GRID_MIN_PIECES) return RD_OK;
-    for (const rd_pot1& p : h->comp) {
-        bool ok = p.force_const > 0.0f && std::isfinite(p.force_const) && std::isfinite(p.radius) && std::isfinite(p.height);
-        for (int d = 0; d < 3; ++d) ok = ok && std::isfinite(p.origin[d]) && std::isfinite(p.normal[d]);
-        if (!ok) return RD_OK;
-    }
-    double lo[3], hi[3], vol = 1.0, reach = 0.0;
+    if (h->comp_sum || h->npieces < min_pieces) return RD_OK;
+    double box[3][2], vol = 1.0, reach = 0.0;
+    union_box(h, box);
+    bool same = h->comp_grid_set;
     for (int d = 0; d < 3; ++d) {
-        lo[d] = h->reps.empty() ? h->prm.lattice_bounds[2 * d] : h->reps[0].lo[d];
-        hi[d] = h->reps.empty() ? h->prm.lattice_bounds[2 * d + 1] : h->reps[0].hi[d];
-        for (const rd_system::Rep& r : h->reps) { lo[d] = std::min(lo[d], r.lo[d]); hi[d] = std::max(hi[d], r.hi[d]); }
-        vol *= hi[d] - lo[d];
+        vol *= box[d][1] - box[d][0];
+        same = same && h->comp_lo[d] == box[d][0] && h->comp_hi[d] == box[d][1];
+    }
+    if (same) { *g = h->comp_built; return RD_OK; }
+    h->comp_passes += passes;
+    if (h->comp_passes <= RD_GRID_PASSES) return RD_OK;
+    // (of pieces and boxes that no grid serves, one without lists is kept)
+    h->comp_grid_set = false;
+    bool ok = true;
+    for (const rd_pot1& p : h->comp) {
+        ok = ok && p.force_const > 0.0f && std::isfinite(p.force_const) && std::isfinite(p.radius) && std::isfinite(p.height);
+        for (int d = 0; d < 3; ++d) ok = ok && std::isfinite(p.origin[d]) && std::isfinite(p.normal[d]);
     }
     const double edge = std::cbrt(vol / RD_GRID_CELLS);
     long cells = 1;
     for (int d = 0; d < 3; ++d) {
-        g->n[d] = (int)std::min(std::max((hi[d] - lo[d]) / edge, 1.0), (double)RD_GRID_CELLS);
+        const double lo = box[d][0], hi = box[d][1];
+        g->n[d] = (int)std::min(std::max((hi - lo) / edge, 1.0), (double)RD_GRID_CELLS);
         cells *= g->n[d];
-        g->lo[d] = (float)lo[d];
-        g->edge[d] = (float)((hi[d] - lo[d]) / g->n[d]);
-        g->inv[d] = (float)(g->n[d] / (hi[d] - lo[d]));
+        g->lo[d] = (float)lo;
+        g->edge[d] = (float)((hi - lo) / g->n[d]);
+        g->inv[d] = (float)(g->n[d] / (hi - lo));
         // the largest separation of a position and a piece, for the rounding margin
         for (const rd_pot1& p : h->comp)
-            reach = std::max(reach, std::max(std::fabs(lo[d] - p.origin[d]), std::fabs(hi[d] - p.origin[d])) +
-                                        std::max(std::fabs(lo[d]), std::fabs(hi[d])) + std::fabs(p.radius) +
+            reach = std::max(reach, std::max(std::fabs(lo - p.origin[d]), std::fabs(hi - p.origin[d])) +
+                                        std::max(std::fabs(lo), std::fabs(hi)) + std::fabs(p.radius) +
                                         std::fabs(p.height));
     }
-    if (cells > 4L * RD_GRID_CELLS || !(reach < 1e12)) { g->list = nullptr; return RD_OK; }
-    if (cells > h->comp_cells) {
-        if (h->d_comp_list) (void)hipFree(h->d_comp_list);
-        h->d_comp_list = nullptr;
-        h->comp_cells = 0;
-        h->comp_grid_set = false;
-        SHIPCK(h, hipMalloc(&h->d_comp_list, sizeof(uint16_t) * RD_GRID_LIST * (size_t)cells));
-        h->comp_cells = cells;
+    if (ok && cells <= 4L * RD_GRID_CELLS && reach < 1e12) {
+        if (cells > h->comp_cells) {
+            if (h->d_comp_list) (void)hipFree(h->d_comp_list);
+            h->d_comp_list = nullptr;
+            h->comp_cells = 0;
+            SHIPCK(h, hipMalloc(&h->d_comp_list, sizeof(uint16_t) * RD_GRID_LIST * (size_t)cells));
+            h->comp_cells = cells;
+        }
+        g->list = h->d_comp_list;
+        hipLaunchKernelGGL(k_comp_grid, dim3((unsigned)((cells + 255) / 256)), dim3(256), pieces_lds(h), h->stream, *g,
+                           (float)(1e-5 * reach), (const RdPiece*)h->d_pieces, h->npieces, h->d_comp_list);
+        SHIPCK(h, hipGetLastError());
     }
-    bool same = h->comp_grid_set;
-    for (int d = 0; d < 3; ++d) same = same && h->comp_lo[d] == lo[d] && h->comp_hi[d] == hi[d];
-    g->list = h->d_comp_list;
-    if (same) return RD_OK;
-    hipLaunchKernelGGL(k_comp_grid, dim3((unsigned)((cells + 255) / 256)), dim3(256), pieces_lds(h), h->stream, *g,
-                       (float)(1e-5 * reach), (const RdPiece*)h->d_pieces, h->npieces, h->d_comp_list);
-    SHIPCK(h, hipGetLastError());
-    for (int d = 0; d < 3; ++d) { h->comp_lo[d] = lo[d]; h->comp_hi[d] = hi[d]; }
+    h->comp_built = *g;
+    for (int d = 0; d < 3; ++d) { h->comp_lo[d] = box[d][0]; h->comp_hi[d] = box[d][1]; }
     h->comp_grid_set = true;
+    h->comp_passes = 0;
     return RD_OK;
 }
 
@@ -1257,16 +1292,25 @@ void rd_host_launch_ext(rd_system* h)
     }
 }
 
+// before steps or gradients that make the external pass `passes` times: the
+// pass takes the grid if it is there or is built now (`changed`: from now on)
+int rd_host_ext_passes(rd_system* h, long passes, bool* changed)
+{
+    if (!h->ext_active() || h->ext_mode != RD_EXT_EXACT || (h->comp_mask & all_types(h)) != all_types(h) || h->comp_near.list)
+        return RD_OK;
+    const int rc = comp_grid(h, &h->comp_near, passes * passes_of(h->n), RD_GRID_SLOT_PIECES);
+    if (changed) *changed = h->comp_near.list != nullptr;
+    return rc;
+}
+
 // gext buffer sized for the current particle count; resident workgroups of
 // the slot passes for the current piece count
 int rd_host_ext_capacity(rd_system* h)
 {
     if (!h->ext_active()) return RD_OK;
     h->comp_near.list = nullptr;
-    if (h->ext_mode == RD_EXT_EXACT && (h->comp_mask & all_types(h)) == all_types(h)) {
-        const int rc = comp_grid(h, &h->comp_near);
-        if (rc) return rc;
-    }
+    const int rc = rd_host_ext_passes(h, 0, nullptr);
+    if (rc) return rc;
     int per = 0;
     SHIPCK(h, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)slots_kernel(h), 256,
                                                            pieces_lds(h)));
@@ -1328,6 +1372,7 @@ extern "C" int rd_set_composite(rd_system* h, int n_pieces, const rd_pot1* piece
         SHIPCK(h, hipMemcpy(h->d_pieces, pc.data(), sizeof(RdPiece) * n_pieces, hipMemcpyHostToDevice));
     }
     h->comp_grid_set = false;
+    h->comp_passes = 0;
     h->comp_allz = std::all_of(pc.begin(), pc.end(), [](const RdPiece& p) { return p.zaxis != 0; });
     h->npieces = n_pieces;
     h->comp_mask = type_mask;
@@ -1386,7 +1431,7 @@ extern "C" int rd_composite_eval(rd_system* h, long m, const float* xyz, float* 
     if (m == 0) return RD_OK;
     SHIPCK(h, hipSetDevice(h->dev));
     RdCompGrid g;
-    const int rc = comp_grid(h, &g);
+    const int rc = comp_grid(h, &g, passes_of(m), RD_GRID_POINT_PIECES);
     if (rc) return rc;
     float *dx = nullptr, *dg = nullptr;                 // positions; gradients, then energies
     SHIPCK(h, hipMalloc(&dx, sizeof(float) * 3 * m));
@@ -1526,10 +1571,20 @@ static int launch_sur_data(rd_system* h, long m, uint64_t seed, float4* xn, floa
     const RdMlpNorm& nm = h->mlp_norm;
     float span[3];
     for (int d = 0; d < 3; ++d) span[d] = (float)(h->norm_hi[d] - nm.lo[d]);
+    // Where more than a few samples fall outside the boxes nearly every wave scans
+    // (a wave of 64 has all inside once in two at 1.1% outside), and no grid is
+    // built for them; the scan of the grid's kernel is taken all the same.
+    double box[3][2], in = 1.0;
+    union_box(h, box);
+    for (int d = 0; d < 3; ++d) {
+        const double lo = nm.lo[d], hi = h->norm_hi[d];
+        in *= std::max(0.0, std::min(hi, box[d][1]) - std::max(lo, box[d][0])) / (hi - lo);
+    }
+    const bool inside = in >= 0.99;
     RdCompGrid g;
-    const int rc = comp_grid(h, &g);
+    const int rc = comp_grid(h, &g, inside ? passes_of(m) : 0, RD_GRID_POINT_PIECES);
     if (rc) return rc;
-    if (g.list)
+    if (g.list || (!inside && !h->comp_sum && h->npieces >= RD_GRID_POINT_PIECES))
         hipLaunchKernelGGL((k_sur_data<false, true>), dim3(nb256(m)), dim3(256), 0, h->stream, m, seed, nm, span[0],
                            span[1], span[2], g, (const RdPiece*)h->d_pieces, h->npieces, xn, tg, bsum);
     else

@@ -1875,7 +1875,16 @@ extern "C" int rd_initialize(rd_system* h)
     rc = upload(h);
     if (rc) return rc;
     h->initialized = true;
-    return RD_OK;
+    return rd_host_passes(h, RD_GRID_NOW);
+}
+
+// passes of the external potential that a call is about to make
+int rd_host_passes(rd_system* h, long passes)
+{
+    bool changed = false;
+    const int rc = rd_host_ext_passes(h, passes, &changed);
+    if (changed) drop_graph(h);      // the captured steps hold the other kernel
+    return rc;
 }
 
 static int refresh(rd_system* h)
@@ -1939,6 +1948,7 @@ extern "C" int rd_simulate(rd_system* h, int nsteps)
 {
     if (!h || nsteps < 0) return RD_EINVAL;
     int rc = refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, nsteps > 0 ? nsteps : RD_GRID_NOW);
     if (rc) return rc;
     if (nsteps == 0) return RD_OK;
     rc = launch_steps(h, nsteps);
@@ -2064,6 +2074,8 @@ extern "C" int rd_gradients(rd_system* h, float* grad, double* energy)
     // hold the particles as last copied out)
     float* const d_grad = (float*)h->d_pn;
     HIPCK(h, hipMemsetAsync(d_etot, 0, sizeof(double), h->stream));
+    rc = rd_host_passes(h, 1);
+    if (rc) return rc;
     if (h->ext_active()) rd_host_launch_ext(h);
     if (h->nwaves <= 3 * h->ncu)     // the line of lanes_per_particle
         hipLaunchKernelGGL((k_gradients_spread<9>), dim3(std::max(1, h->nwaves)), dim3(64 * 9), 0, h->stream, h->d_ps,
@@ -2639,6 +2651,7 @@ extern "C" int rd_simulate_async(rd_system* h, int nsteps)
 {
     if (!h || nsteps < 0) return RD_EINVAL;
     int rc = refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, nsteps > 0 ? nsteps : RD_GRID_NOW);
     if (rc) return rc;
     return nsteps > 0 ? launch_steps(h, nsteps) : RD_OK;
 }

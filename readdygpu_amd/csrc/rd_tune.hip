@@ -39,6 +39,7 @@ extern "C" int rd_autotune(rd_system* h, int trial_steps, double* best_ms)
 {
     if (!h || trial_steps < 1) return RD_EINVAL;
     int rc = rd_host_refresh(h);
+    if (rc == RD_OK) rc = rd_host_passes(h, RD_GRID_NOW);
     if (rc) return rc;
     if (h->n == 0) { if (best_ms) *best_ms = 0.0; return RD_OK; }
     // snapshot: positions (index order) and the step counter

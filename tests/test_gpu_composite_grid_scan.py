@@ -27,7 +27,7 @@ def test_scans(make, n):
             x[m // 2] = np.float32(BOX)                  # the domain's upper corner
             grad, best = scan(sim, pieces, x)
             sim.set_composite(pieces)
-            for _ in range(3):
+            for _ in range(5):                           # before and after the lists are built
                 g, e = sim.composite_eval(x)
                 assert np.array_equal(e, best) and np.array_equal(g, grad), m
         # the step's pass, particles that do not fill the last wave
@@ -53,7 +53,7 @@ def test_data_wider_than_the_boxes():
             sim.set_composite(pieces)
             sim.surrogate_init(3)
             sim.set_surrogate_norm((0, 0, 0), tuple(2.5 * v for v in BOX), 1.0)
-            for _ in range(3):
+            for _ in range(5):                       # before and after the lists are built
                 r = [sim.surrogate_make_data(70_001, seed=4), sim.surrogate_validate(10_001, seed=5)]
                 out.append(r)
     assert all(r == out[0] for r in out), out

@@ -32,7 +32,7 @@ def compare(box, pieces, seed, m=60_000):
     with Simulation(spec, (xyz * np.float32(0.2)).astype(np.float32), types) as sim:
         grad, best = scan(sim, pieces, x)
         sim.set_composite(pieces)
-        for _ in range(4):                     # before and after the lists are built
+        for _ in range(5):                     # before and after the lists are built
             g, e = sim.composite_eval(x)
             assert np.array_equal(e, best)
             assert np.array_equal(g, grad)
