@@ -204,6 +204,7 @@ struct rd_system {
 };
 
 #define RD_STAGE_MAX ((size_t)4 << 20)
+#define RD_STAGE_MIN ((size_t)64 << 10)     // least size of a buffer
 char* rd_host_stage(rd_system* h, size_t bytes);
 double rd_host_r0(const rd_system* h, int i, int j);
 int rd_host_refresh(rd_system* h);

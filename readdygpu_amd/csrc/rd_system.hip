@@ -998,7 +998,7 @@ char* rd_host_stage(rd_system* h, size_t bytes)
             return h->hp_stage;
         }
     }
-    const size_t cap = std::min(std::max(bytes + bytes / 4, (size_t)64 << 10), RD_STAGE_MAX);
+    const size_t cap = std::min(std::max(bytes + bytes / 4, RD_STAGE_MIN), RD_STAGE_MAX);
     if (hipHostMalloc((void**)&h->hp_stage, cap, hipHostMallocDefault) != hipSuccess) {
         h->hp_stage = nullptr;
         (void)hipGetLastError();
