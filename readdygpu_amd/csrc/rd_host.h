@@ -142,7 +142,7 @@ struct rd_system {
     struct Graph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
-        int asked = 0;
+        bool asked = false;
     };
     std::map<int, Graph> graphs;
 
