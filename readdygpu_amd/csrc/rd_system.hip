@@ -2222,10 +2222,18 @@ static hipError_t launch_rdf_form(rd_system* h, int S, const RdRdf& rdf, size_t 
 // through the uncut half stencil with two atomics a pair: 461), 50,000
 // 54 / 46 / 59 (132), 200,000 134 / 85 / 82 (152), 1M 555 / 284 / 227 (321),
 // 64 replicas of 911,000 particles 665 / 399 / 338 (620).
+// A histogram (types x types x bins) beyond 32 KB leaves room for four or fewer
+// workgroups of 256 threads on a compute unit, and its clearing and flush weigh
+// more than the 128 particles it is for: 2 lanes in 1,024 threads, 512 particles.
+// 1M particles at 1e-2 per nm^3, 6 nm, 8 types, 256 / 1,024 threads: 100 bins
+// (25.6 KB) 186 / 124 us, 130 189 / 129, 200 241 / 140, 630 853 / 225; 262,145
+// particles at 1e-3, 20 nm: 100 bins 172 / 193, 130 199 / 195, 630 587 / 278.
+#define RD_RDF_WIDE ((size_t)32 << 10)
 static hipError_t launch_rdf(rd_system* h, int S, const RdRdf& rdf, size_t lds, long total)
 {
     if (h->nwaves <= 2 * h->ncu) return launch_rdf_form<1024, 16, 4>(h, S, rdf, lds, total);
     if (h->nwaves <= 16 * h->ncu) return launch_rdf_form<512, 4, 4>(h, S, rdf, lds, total);
+    if (lds > RD_RDF_WIDE) return launch_rdf_form<1024, 2, 2>(h, S, rdf, lds, total);
     return launch_rdf_form<256, 2, 2>(h, S, rdf, lds, total);
 }
 
