@@ -833,8 +833,9 @@ struct RdWaveLds {
 //   the 64 lanes for evaluation, which adds a pair's term to its home's sums in
 //   LDS (integers: the order does not matter).  With each lane evaluating its
 //   own hits, the interaction code runs as often as the lane with the most hits
-//   needs (vector instructions bound this kernel: 91% busy in the cytosol), and
-//   a lane with more than its list holds sends the wave into a second walk;
+//   needs, and a lane with more than its list holds sends the wave into a second
+//   walk (vector instructions bound this kernel: with the hits dealt they issue
+//   in 88% of its cycles in the cytosol, 90% of their lanes at work);
 // - a row's two runs are walked as one sequence per lane, so that a wave
 //   iterates over the largest sum of a lane's runs, not over the largest first
 //   run and then the largest second one (16 to 19% fewer slots in lattices of
